@@ -7,7 +7,8 @@ import sys
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 SRCS = [os.path.join(HERE, "csrc", f) for f in ("m3d_elastic.hip", "m3d_thermal.hip", "m3d_basic.hip", "m3d_rec.hip",
-                                                   "m3d_gen.hip", "m3d_2d.hip", "m3d_perc.hip")]
+                                                   "m3d_gen.hip", "m3d_2d.hip", "m3d_perc.hip",
+                                                   "m3d_flex.hip", "m3d_flex_basic.hip")]
 LIB = os.path.join(HERE, "libmat3d.so")
 
 HIPCC_FLAGS = [
@@ -24,7 +25,7 @@ HIPCC_FLAGS = [
 
 
 def build(verbose: bool = False, out: str | None = None, defines: list[str] | None = None) -> str:
-    """Compile the three units in parallel, then link libmat3d.so (or
+    """Compile the units in parallel, then link libmat3d.so (or
     ``out``); ``defines`` are extra -D macros (tuning parameters)."""
     hipcc = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
     lib = out or LIB

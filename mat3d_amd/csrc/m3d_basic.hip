@@ -2,8 +2,8 @@
 // mixed control and the J2 / damage updates (runAnalysis "ep" / "ed",
 // src/3d/FFT_analysis3D.cpp:796-853), in FP64 and FP32.  The host driver is BasicRunner
 // (m3d_basic_host.hpp); it calls the launchers at the end of this file for
-// grids whose line lengths have specialised kernels and the runtime-planned
-// kernels of m3d_basic.hpp otherwise.
+// grids whose line lengths have specialised kernels and those of
+// m3d_flex_basic.hip otherwise.
 #include "m3d_basic_fast.hpp"
 
 #include <stdexcept>

@@ -2,16 +2,17 @@
 // J2 / damage constitutive updates: runAnalysis "ep" / "ed",
 // src/3d/FFT_analysis3D.cpp:796-853.
 //
-// Per iteration (one stage = four kernels + two finalisers):
-//   zb   : c2r along z of eps^ (6 comps) -> eps;  constitutive() -> sigma
+// Per iteration (one stage = four kernels + three finalisers; m3d_basic.hip
+// and m3d_flex_basic.hip hold the kernels):
+//   z    : c2r along z of eps^ (6 comps) -> eps;  constitutive() -> sigma
 //          (elastoPlastic :640-691 or elastoDamage :619-638, per voxel,
 //          history in HBM); FP64 partial sums of every component of sigma and
-//          eps (updateE :583-594 needs the means); r2c along z of sigma and
-//          eps -> a 12-component half spectrum [sigma^ | eps^]
+//          eps (updateE :583-594 needs the means); r2c along z of sigma (and,
+//          in the start stage, of eps)
 //   fin1 : itNo, diff_sum_field (:399, with the E of the Green step that made
 //          this iterate), updateE -> E for the next Green step
-//   y    : forward FFT along y (12 components)
-//   xb   : forward FFT along x; eqVar partials from sigma^ (convergenceCheck
+//   y    : forward FFT along y
+//   x    : forward FFT along x; eqVar partials from sigma^ (convergenceCheck
 //          :351-389 -- the reference transforms sigma once more for it, here it
 //          is the spectrum the next Green step uses anyway); Green step
 //          t3 = eps^ - Gamma0:sigma^ (multiplyGF :323-338), DC = E N; inverse
@@ -26,7 +27,7 @@
 namespace m3d {
 
 enum { BEH_EP = 1, BEH_ED = 2 };
-// FINAL (specialised kernels only): the fields and state of the last iterate
+// FINAL: the fields and state of the last iterate
 // of an increment, recomputed from the Green output its z pass read (the
 // FP64 iterations do not write them)
 enum { BMODE_START = 0, BMODE_ITER = 1, BMODE_RESTART = 2, BMODE_FINAL = 3 };
@@ -42,15 +43,14 @@ struct BPtr {
     T* phi;          // N   yield function of the last constitutive call ("ep")
     T* dep;          // N   plastic multiplier increment ("ep")
     T* seff;         // N   von Mises stress after the return map ("ep")
-    T* sig_star;     // 6N  sigma_old - C eps_old, once per increment ("ep", FP64 specialised kernels)
-    double* pfin;    // [14][nbz] block sums of the fused FINAL pass ("ep", FP64 specialised kernels)
+    T* sig_star;     // 6N  sigma_old - C eps_old, once per increment ("ep", FP64)
+    double* pfin;    // [14][nbz] block sums of the fused FINAL pass ("ep", FP64)
     long long sU;    // per-solve stride of the 6N fields
     long long sN;    // per-solve stride of the N fields
     cx<T>* S6;       // Green output, 6 components (read by the z pass)
-    cx<T>* S12;      // [sigma^ | eps^], 12 components (generic kernels, START)
-                     // or sigma^, 6 components (specialised ITER)
-    cx<T>* S6w;      // Green output written by the specialised x pass (the other S6 buffer)
-    cx<T>* Eh;       // eps^ after the Green step, tile order of the specialised x pass
+    cx<T>* S12;      // [sigma^ | eps^], 12 components (START) or sigma^, 6 components (ITER)
+    cx<T>* S6w;      // Green output written by the x pass (the other S6 buffer)
+    cx<T>* Eh;       // eps^ after the Green step (specialised x pass: in its tile order)
     long long sS6, sS12;
     const uint8_t* ph;
     const double* mat; // per phase {la, mu, Sy, H, n, P, Y0, 0}
@@ -161,294 +161,6 @@ __device__ __forceinline__ void damage_update(const double* m, const T* eps, T& 
     }
 #pragma unroll
     for (int k = 0; k < 6; ++k) sig[k] = (T(1) - d) * c[k];
-}
-
-// ------------------------------------------------------------------- z pass
-// Block: solve s, plane x, lines y0..y0+TY-1; LDS lines l = yl*12 + c
-// (c < 6: sigma, c >= 6: eps), each lsz complex.
-template <typename T, int BEH, int MODE, bool GEN>
-__global__ void __launch_bounds__(ZTHREADS) k_zbasic(Geo g, BPtr<T> p)
-{
-    extern __shared__ __align__(16) unsigned char smem_raw[];
-    __shared__ double red[ZTHREADS / 64];
-    constexpr int C = 12;
-    cx<T>* sl = reinterpret_cast<cx<T>*>(smem_raw);
-    T* sr = reinterpret_cast<T*>(smem_raw);
-    const int per = g.Nx * g.nty;
-    const int s = blockIdx.x / per;
-    const int t = blockIdx.x % per;
-    const int x = t / g.nty;
-    const int y0 = (t % g.nty) * g.TY;
-    Ctl& ctl = p.ctl[s];
-    if (ctl.done) return;
-    const int Nz = g.Nz, Nzh = g.Nzh, lsz = g.lsz, TY = g.TY;
-    const long long vox0 = ((long long)x * g.Ny + y0) * Nz;
-    const int tid = threadIdx.x, nthr = blockDim.x;
-
-    T* eps = p.eps + (long long)s * p.sU + vox0 * 6;
-    T* sig = p.sig + (long long)s * p.sU + vox0 * 6;
-    const uint8_t* ph = p.ph + vox0;
-
-    if (MODE == BMODE_ITER) {
-        // Green output (6 comps) -> lines yl*12 + 6 + c
-        const cx<T>* src = p.S6 + (long long)s * p.sS6 + ((long long)x * g.Ny + y0) * Nzh * 6;
-        const int tot = TY * Nzh * 6;
-        for (int e = tid; e < tot; e += nthr) {
-            const int yl = e / (Nzh * 6);
-            const int r = e - yl * Nzh * 6;
-            const int kz = r / 6, c = r - kz * 6;
-            sl[(yl * C + 6 + c) * lsz + kz] = src[e];
-        }
-        __syncthreads();
-        const LineGeo lg6{TY * 6, 6, lsz, C * lsz, 1};
-        cx<T>* s6 = sl + 6 * lsz;
-        if (g.zeven) {
-            const int L = Nz / 2;
-            const int half = L / 2 + 1;
-            for (int e = tid; e < TY * 6 * half; e += nthr) {
-                const int l = e / half, k = e - l * half;
-                cx<T>* ln = s6 + lg6.off(l);
-                if (k == 0) {
-                    const T x0 = ln[0].re, xl = ln[L].re;
-                    ln[0] = cx<T>{x0 + xl, x0 - xl};
-                } else {
-                    const int kk = L - k;
-                    const cx<T> Xk = ln[k], Xc = ln[kk];
-                    cx<T> w = p.twz[k];
-                    w.im = -w.im;
-                    ln[k] = (Xk + cconj(Xc)) + rot90<1>(cmul(w, Xk - cconj(Xc)));
-                    if (kk != k) {
-                        cx<T> w2 = p.twz[kk];
-                        w2.im = -w2.im;
-                        ln[kk] = (Xc + cconj(Xk)) + rot90<1>(cmul(w2, Xc - cconj(Xk)));
-                    }
-                }
-            }
-            __syncthreads();
-            fft_lines<T, 1, EPT, false, GEN>(s6, lg6, g.az, p.twz);
-        } else {
-            for (int e = tid; e < TY * 6 * Nzh; e += nthr) {
-                const int l = e / Nzh, k = e - l * Nzh;
-                cx<T>* ln = s6 + lg6.off(l);
-                if (k == 0) ln[0].im = T(0);
-                else ln[Nz - k] = cconj(ln[k]);
-            }
-            __syncthreads();
-            fft_lines<T, 1, EPT, false, GEN>(s6, lg6, g.az, p.twz);
-            // compact real parts into the real view of each line
-            for (int l = 0; l < TY * 6; ++l) {
-                cx<T>* ln = s6 + lg6.off(l);
-                T* rl = reinterpret_cast<T*>(ln);
-                T v[EPT];
-#pragma unroll
-                for (int i = 0; i < EPT; ++i) {
-                    const int z = tid + i * nthr;
-                    if (z < Nz) v[i] = ln[z].re;
-                }
-                __syncthreads();
-#pragma unroll
-                for (int i = 0; i < EPT; ++i) {
-                    const int z = tid + i * nthr;
-                    if (z < Nz) rl[z] = v[i];
-                }
-                __syncthreads();
-            }
-        }
-    }
-
-    // constitutive update per voxel
-    double acc[NBSUM];
-#pragma unroll
-    for (int q = 0; q < NBSUM; ++q) acc[q] = 0.0;
-    bool bad = false;
-    const int nv = TY * Nz;
-    for (int v = tid; v < nv; v += nthr) {
-        const int yl = v / Nz, z = v - yl * Nz;
-        const int k = ph[v];
-        const double* m = p.mat + k * 8;
-        T e[6], sg[6];
-        if (MODE == BMODE_ITER) {
-            const T invN = T(1); // the Green step already divided by N
-#pragma unroll
-            for (int c = 0; c < 6; ++c) e[c] = sr[(yl * C + 6 + c) * 2 * lsz + z] * invN;
-#pragma unroll
-            for (int c = 0; c < 6; ++c) eps[(long long)v * 6 + c] = e[c];
-        } else {
-#pragma unroll
-            for (int c = 0; c < 6; ++c) e[c] = eps[(long long)v * 6 + c];
-        }
-        const long long vg = vox0 + v;
-        if (BEH == BEH_EP) {
-            T so[6], eo[6], phi, dep, seff;
-#pragma unroll
-            for (int c = 0; c < 6; ++c) {
-                so[c] = p.sig_old[(long long)s * p.sU + vg * 6 + c];
-                eo[c] = p.eps_old[(long long)s * p.sU + vg * 6 + c];
-            }
-            const T epe = p.ep[(long long)s * p.sN + vg];
-            if (!j2_update<T>(m, e, eo, so, epe, sg, phi, dep, seff)) bad = true;
-            p.phi[(long long)s * p.sN + vg] = phi;
-            p.dep[(long long)s * p.sN + vg] = dep;
-            p.seff[(long long)s * p.sN + vg] = seff;
-        } else {
-            T d = p.ep[(long long)s * p.sN + vg];
-            damage_update<T>(m, e, d, sg);
-            p.ep[(long long)s * p.sN + vg] = d;
-        }
-#pragma unroll
-        for (int c = 0; c < 6; ++c) {
-            sig[(long long)v * 6 + c] = sg[c];
-            acc[c] += (double)sg[c];
-            acc[6 + c] += (double)e[c];
-            sr[(yl * C + c) * 2 * lsz + z] = sg[c];
-            sr[(yl * C + 6 + c) * 2 * lsz + z] = e[c];
-        }
-    }
-    if (bad) ctl.err = 1;
-#pragma unroll
-    for (int q = 0; q < NBSUM; ++q) {
-        const double bs = block_sum(acc[q], red);
-        if (tid == 0) p.psum[((long long)s * NBSUM + q) * g.nbz + t] = bs;
-    }
-    __syncthreads();
-
-    // forward r2c of all 12 components
-    const LineGeo lg{TY * C, TY * C, lsz, 0, 1};
-    if (g.zeven) {
-        fft_lines<T, -1, EPT, false, GEN>(sl, lg, g.az, p.twz);
-        const int L = Nz / 2;
-        const int half = L / 2 + 1;
-        for (int e = tid; e < TY * C * half; e += nthr) {
-            const int l = e / half, k = e - l * half;
-            cx<T>* ln = sl + l * lsz;
-            if (k == 0) {
-                const cx<T> z0 = ln[0];
-                ln[0] = cx<T>{z0.re + z0.im, T(0)};
-                ln[L] = cx<T>{z0.re - z0.im, T(0)};
-            } else {
-                const int kk = L - k;
-                const cx<T> zk = ln[k], zc = cconj(ln[kk]);
-                const cx<T> E = cscale(zk + zc, T(0.5));
-                const cx<T> O = cscale(rot90<-1>(zk - zc), T(0.5));
-                ln[k] = E + cmul(p.twz[k], O);
-                if (kk != k) ln[kk] = cconj(E) + cmul(p.twz[kk], cconj(O));
-            }
-        }
-        __syncthreads();
-    } else {
-        for (int l = 0; l < TY * C; ++l) {
-            cx<T>* ln = sl + l * lsz;
-            const T* rl = reinterpret_cast<const T*>(ln);
-            T v[EPT];
-#pragma unroll
-            for (int i = 0; i < EPT; ++i) {
-                const int z = tid + i * nthr;
-                if (z < Nz) v[i] = rl[z];
-            }
-            __syncthreads();
-#pragma unroll
-            for (int i = 0; i < EPT; ++i) {
-                const int z = tid + i * nthr;
-                if (z < Nz) ln[z] = cx<T>{v[i], T(0)};
-            }
-            __syncthreads();
-        }
-        fft_lines<T, -1, EPT, false, GEN>(sl, lg, g.az, p.twz);
-    }
-    cx<T>* dst = p.S12 + (long long)s * p.sS12 + ((long long)x * g.Ny + y0) * Nzh * C;
-    const int tot = TY * Nzh * C;
-    for (int e = tid; e < tot; e += nthr) {
-        const int yl = e / (Nzh * C);
-        const int r = e - yl * Nzh * C;
-        const int kz = r / C, c = r - kz * C;
-        dst[e] = sl[(yl * C + c) * lsz + kz];
-    }
-}
-
-// --------------------------------------------------------------- x pass
-// Block: solve s, row y, kz tile; LDS [x][kzl*12 + c] (12 comps in, 6 out).
-template <typename T, bool GEN>
-__global__ void __launch_bounds__(XYTHREADS) k_xbasic(Geo g, BPtr<T> p)
-{
-    extern __shared__ __align__(16) unsigned char smem_raw[];
-    __shared__ double red[XYTHREADS / 64];
-    constexpr int C = 12;
-    cx<T>* sl = reinterpret_cast<cx<T>*>(smem_raw);
-    const int per = g.Ny * g.nkx;
-    const int s = blockIdx.x / per;
-    const int t = blockIdx.x % per;
-    const int y = t / g.nkx;
-    const int kz0 = (t % g.nkx) * g.TKx;
-    const Ctl& ctl = p.ctl[s];
-    if (ctl.done) return;
-    const int nk = min(g.TKx, g.Nzh - kz0);
-    const int w = nk * C;
-    const cx<T>* base = p.S12 + (long long)s * p.sS12 + ((long long)y * g.Nzh + kz0) * C;
-    const long long xstride = (long long)g.Ny * g.Nzh * C;
-    const int tot = g.Nx * w;
-    for (int e = threadIdx.x; e < tot; e += blockDim.x) {
-        const int xx = e / w, r = e - xx * w;
-        sl[e] = base[xx * xstride + r];
-    }
-    __syncthreads();
-    fft_lines<T, -1, EPT, true, GEN>(sl, LineGeo{w, w, 1, 0, w}, g.ax, p.twx);
-    const T la0 = T(ctl.la0), mu0 = T(ctl.mu0);
-    double acc = 0.0;
-    for (int f = threadIdx.x; f < g.Nx * nk; f += blockDim.x) {
-        const int kx = f / nk, kzl = f - kx * nk;
-        const int kz = kz0 + kzl;
-        cx<T>* v = sl + kx * w + kzl * C;
-        // eqVar partial from sigma^ (kz >= 1), dd at DC
-        double a2[6];
-#pragma unroll
-        for (int c = 0; c < 6; ++c) a2[c] = (double)v[c].re * (double)v[c].re + (double)v[c].im * (double)v[c].im;
-        if (kz >= 1) {
-            const double z0 = Elastic::fmap(kz, g.Nz), z1 = Elastic::fmap(y, g.Ny), z2 = Elastic::fmap(kx, g.Nx);
-            const double q = a2[0] * z0 * z0 + a2[1] * z1 * z1 + a2[2] * z2 * z2 + a2[3] * ((z1 + z1) + (z2 + z2)) +
-                             a2[4] * ((z0 + z0) + (z2 + z2)) + a2[5] * ((z0 + z0) + (z1 + z1));
-            acc += sqrt(fabs(q));
-        }
-        if (kx == 0 && y == 0 && kz == 0) {
-            p.pchk[(long long)s * (g.nbx + 1) + g.nbx] = sqrt(a2[0] + a2[1] + a2[2] + 2 * a2[3] + 2 * a2[4] + 2 * a2[5]);
-#pragma unroll
-            for (int c = 0; c < 6; ++c) v[c] = cx<T>{T(ctl.E[c]), T(0)};
-        } else {
-            // t3 = eps^ - Gamma0:sigma^ (Nyquist planes: Hermitian part of the Gamma0 term)
-            int fz = Elastic::fmap(kz, g.Nz), fy = Elastic::fmap(y, g.Ny), fxx = Elastic::fmap(kx, g.Nx);
-            T xi[3] = {T(fz), T(fy), T(fxx)};
-            cx<T> sg[6], o[6];
-#pragma unroll
-            for (int c = 0; c < 6; ++c) sg[c] = v[c];
-            green_elastic<T>(xi, sg, o, 1, la0, mu0);
-            const bool plane = (kz == 0) || (g.zeven && kz == g.Nz / 2);
-            if (plane) {
-                const int px = (g.Nx - kx) % g.Nx, py = (g.Ny - y) % g.Ny;
-                const int gz = Elastic::fmap(kz, g.Nz), gy = Elastic::fmap(py, g.Ny), gx = Elastic::fmap(px, g.Nx);
-                if (gz != -fz || gy != -fy || gx != -fxx) {
-                    T xp[3] = {T(gz), T(gy), T(gx)};
-                    cx<T> o2[6];
-                    green_elastic<T>(xp, sg, o2, 1, la0, mu0);
-#pragma unroll
-                    for (int c = 0; c < 6; ++c) o[c] = cscale(o[c] + o2[c], T(0.5));
-                }
-            }
-            const T sc = T(g.invN);
-#pragma unroll
-            for (int c = 0; c < 6; ++c) v[c] = cscale(v[6 + c] - o[c], sc);
-        }
-    }
-    const double bs = block_sum(acc, red);
-    if (threadIdx.x == 0) p.pchk[(long long)s * (g.nbx + 1) + t] = bs;
-    __syncthreads();
-    fft_lines<T, 1, EPT, true, GEN>(sl, LineGeo{nk * 6, 6, 1, C, w}, g.ax, p.twx);
-    cx<T>* ob = p.S6 + (long long)s * p.sS6 + ((long long)y * g.Nzh + kz0) * 6;
-    const long long ostride = (long long)g.Ny * g.Nzh * 6;
-    const int tot6 = g.Nx * nk * 6;
-    for (int e = threadIdx.x; e < tot6; e += blockDim.x) {
-        const int xx = e / (nk * 6), r = e - xx * nk * 6;
-        const int kzl = r / 6, c = r - kzl * 6;
-        ob[xx * ostride + r] = sl[xx * w + kzl * C + c];
-    }
 }
 
 // ----------------------------------------------------------- finalisers
@@ -635,8 +347,8 @@ __global__ void __launch_bounds__(256) k_bfsums(Geo g, const double* pfin, doubl
     if (threadIdx.x == 0) out[(long long)q * nblk + b] = v;
 }
 
-// sigma_star = sigma_old - C eps_old for the next increment's start stage on
-// the specialised FP64 "ep" kernels, after k_bupdate (one solve)
+// sigma_star = sigma_old - C eps_old for the next increment's start stage
+// ("ep", FP64), after k_bupdate (one solve)
 template <typename T>
 __global__ void k_bstar(Geo g, BPtr<T> p)
 {

@@ -1,9 +1,8 @@
 // m3d_basic_fast.hpp -- interface of the compile-time specialised kernels of
 // the basic scheme ("ep" / "ed", FFT_analysis3D.cpp:796-853), defined in
-// m3d_basic.hip.  Same passes as the runtime-planned kernels of
-// m3d_basic.hpp (z pass with the constitutive update, y pass on 12
-// components, x pass with eqVar partials and the Green step, y pass on 6),
-// with every FFT length and tile a template constant.
+// m3d_basic.hip: z pass with the constitutive update, y pass on 12 (start
+// stage) or 6 components, x pass with eqVar partials and the Green step, y pass
+// on 6, with every FFT length and tile a template constant.
 #pragma once
 #include "m3d_basic.hpp"
 #include "m3d_fast.hpp"
@@ -94,4 +93,13 @@ template <typename T>
 void launch_y6(const Geo& g, const Ptr<T>& p, hipStream_t st);
 
 } // namespace bfast
+
+// The same passes for every other grid, in FP64 (m3d_flex_basic.hip): g is a
+// run-time plan of 12 (start stage) or 6 components (iterations, FINAL) whose
+// z and x tiles plan() has set; the y passes are flex::launch_y.
+namespace bflex {
+void plan(Geo& g);
+void launch_z(int beh, int mode, const Geo& g, const BPtr<double>& p, hipStream_t st, bool lin);
+void launch_x(const Geo& g, const BPtr<double>& p, hipStream_t st, bool e6);
+} // namespace bflex
 } // namespace m3d

@@ -8,24 +8,27 @@ namespace {
 
 // ------------------------------------------------------ basic scheme runner
 // runAnalysis "ep" / "ed" (FFT_analysis3D.cpp:796-853) on one solve.  FP64
-// handles, and grids without specialised kernels, iterate in FP64.  On an
+// handles, and grids without the compile-time kernels, iterate in FP64.  On an
 // FP32+polish handle each increment iterates in FP32 (fields, FFTs, return
 // map) until the stop rule holds at polish_factor x tol, then continues in
 // FP64 from the promoted Green output under the reference's rule; the
 // history (sigma_old, eps_old, ep) is kept and updated in FP64.
 struct BasicRunner {
     Engine<Elastic>& e;
-    Geo g12{}, g6{};
+    Geo g12{}, g6{};   // run-time plans of the start stage and of the iterations (m3d_flex_basic.hip)
     Geo gf{};          // tiles of the compile-time specialised kernels
     Geo gf6{};         // the same with the row strides of the 6-component spectrum
     bool fast = false; // grid has specialised basic kernels (m3d_basic.hip)
+    // the z and x tiles of a start stage, and of the iterations and FINAL
+    const Geo& gs() const { return fast ? gf : g12; }
+    const Geo& gi() const { return fast ? gf : g6; }
     int beh;
     bool two = false;       // FP32 phase + FP64 polish per increment
     double* f6 = nullptr;   // eps, sig, sig_old, eps_old, sig_star (5 x 6N)
     double* f1 = nullptr;   // ep|d, phi, dep, seff (4 x N)
-    unsigned char* S6 = nullptr;  // two 6-component spectra: the specialised passes alternate them
+    unsigned char* S6 = nullptr;  // two 6-component spectra: the iterations alternate them
     unsigned char* S12 = nullptr;
-    unsigned char* Eh = nullptr;  // eps^ of the specialised x pass
+    unsigned char* Eh = nullptr;  // eps^ of the x pass
     float* f6s = nullptr;   // FP32 phase: the same fields in FP32
     float* f1s = nullptr;
     unsigned char* S6s = nullptr;
@@ -50,12 +53,13 @@ struct BasicRunner {
     {
         g12 = make_geo<double>(e.Nx, e.Ny, e.Nz, 12);
         g6 = make_geo<double>(e.Nx, e.Ny, e.Nz, 6);
-        g12.fz = g12.fy = g12.fx = 0;
-        g6.fz = g6.fy = g6.fx = 0;
-        // make_geo may have switched tiles to the specialised kernels' shapes
-        plan_tiles(g12, sizeof(cx<double>));
-        plan_tiles(g6, sizeof(cx<double>));
-        g12.nsolve = g6.nsolve = 1;
+        for (Geo* q : {&g12, &g6}) {
+            // make_geo may have switched tiles to the specialised kernels' shapes
+            flex::plan(*q, sizeof(cx<double>));
+            bflex::plan(*q);
+            q->fz = q->fy = q->fx = 0;
+            q->nsolve = 1;
+        }
         // the basic scheme's spectra keep plain [x][y][kz] rows without padding
         for (Geo* q : {&g12, &g6}) {
             q->lxb = q->xbm = 0;
@@ -75,21 +79,19 @@ struct BasicRunner {
             gf6.sy = gf6.sxb = (long long)gf.Nzh * 6;
             gf6.sxa = (long long)gf.Ny * gf6.sy;
         }
-        const int nbz = fast ? std::max(g12.nbz, gf.nbz) : g12.nbz;
-        const int nbx = fast ? std::max(g12.nbx, gf.nbx) : g12.nbx;
+        const int nbz = std::max(gs().nbz, gi().nbz);
+        const int nbx = std::max(gs().nbx, gi().nbx);
         const size_t N = (size_t)e.N, H = (size_t)e.H;
         try {
             e.alloc(&f6, sizeof(double) * 30 * N);
             e.alloc(&f1, sizeof(double) * 4 * N);
             e.alloc(&S6, sizeof(cx<double>) * 12 * H);
             e.alloc(&S12, sizeof(cx<double>) * 12 * H);
-            if (fast) {
-                neh = (size_t)gf.nbx * e.Nx * gf.TKx * 6;
-                e.alloc(&Eh, sizeof(cx<double>) * neh);
-            }
+            neh = fast ? (size_t)gf.nbx * e.Nx * gf.TKx * 6 : (size_t)6 * H;
+            e.alloc(&Eh, sizeof(cx<double>) * neh);
             e.alloc(&psum, sizeof(double) * NBSUM * nbz);
             e.alloc(&psum2, sizeof(double) * NBSUM * BSPLIT);
-            if (fast) e.alloc(&pfin, sizeof(double) * 14 * (size_t)gf.nbz);
+            e.alloc(&pfin, sizeof(double) * 14 * (size_t)gi().nbz);
             e.alloc(&pchk, sizeof(double) * (nbx + 1));
             e.alloc(&bs, sizeof(double) * 14 * nblk);
             e.alloc(&mat, sizeof(double) * 256 * 8);
@@ -127,9 +129,8 @@ struct BasicRunner {
         cx<T>* b = reinterpret_cast<cx<T>*>(sizeof(T) == 8 ? S6 : S6s);
         return b + (half ? 6 * e.H : 0);
     }
-    // par < 0: the generic kernels (one S6 buffer, read and written in place);
-    // par = 0 / 1: the specialised z pass reads S6 buffer par and the x pass
-    // writes buffer 1 - par
+    // par = 0 / 1: the z pass reads S6 buffer par and the x pass writes
+    // buffer 1 - par (par < 0: fields only)
     template <typename T>
     BPtr<T> bptr_t(int par = -1)
     {
@@ -196,61 +197,43 @@ struct BasicRunner {
         hipLaunchKernelGGL((k_bfin1<MODE>), dim3(1), dim3(FTHREADS), 0, e.st, g, ctl, psum2);
     }
 
-    template <bool GEN>
-    void stage(int mode)
-    {
-        hipStream_t st = e.st;
-        BPtr<double> bp = bptr();
-        Ptr<double> yp = yptr();
-        const size_t zsm = (size_t)g12.TY * 12 * g12.lsz * sizeof(cx<double>);
-        const size_t ysm12 = (size_t)g12.Ny * g12.TKy * 12 * sizeof(cx<double>);
-        const size_t ysm6 = (size_t)g6.Ny * g6.TKy * 6 * sizeof(cx<double>);
-        const size_t xsm = (size_t)g12.Nx * g12.TKx * 12 * sizeof(cx<double>);
-        if (mode == BMODE_START) {
-            if (beh == BEH_EP)
-                hipLaunchKernelGGL((k_zbasic<double, BEH_EP, BMODE_START, GEN>), dim3(g12.nbz), dim3(ZTHREADS), zsm, st, g12, bp);
-            else
-                hipLaunchKernelGGL((k_zbasic<double, BEH_ED, BMODE_START, GEN>), dim3(g12.nbz), dim3(ZTHREADS), zsm, st, g12, bp);
-            bfin1<BMODE_START>(g12);
-        } else {
-            if (beh == BEH_EP)
-                hipLaunchKernelGGL((k_zbasic<double, BEH_EP, BMODE_ITER, GEN>), dim3(g12.nbz), dim3(ZTHREADS), zsm, st, g12, bp);
-            else
-                hipLaunchKernelGGL((k_zbasic<double, BEH_ED, BMODE_ITER, GEN>), dim3(g12.nbz), dim3(ZTHREADS), zsm, st, g12, bp);
-            bfin1<BMODE_ITER>(g12);
-        }
-        hipLaunchKernelGGL((k_ypass<double, 12, -1, BUF_K, GEN>), dim3(g12.Nx * g12.nky), dim3(XYTHREADS), ysm12, st, g12, yp);
-        hipLaunchKernelGGL((k_xbasic<double, GEN>), dim3(g12.nbx), dim3(XYTHREADS), xsm, st, g12, bp);
-        hipLaunchKernelGGL((k_bfin2<0>), dim3(1), dim3(FTHREADS), 0, st, g12, ctl, pchk);
-        hipLaunchKernelGGL((k_ypass<double, 6, 1, BUF_MAIN, GEN>), dim3(g6.Nx * g6.nky), dim3(XYTHREADS), ysm6, st, g6, yp);
-    }
-
-    // one stage with the specialised kernels (the sequence of stage()); the
+    // one stage: z pass, sums and updateE, y pass, x pass, stop rule, y pass; the
     // restart stage is a start stage (strain from HBM) that keeps itNo.  A
     // start stage transforms [sigma | eps] and writes S6 buffer 0 (par = 1);
     // an iteration reads S6 buffer par, transforms sigma only (the x pass
     // keeps eps^ in Eh) and writes buffer 1 - par.
     template <typename T = double>
-    void stage_fast(int mode, int par)
+    void stage(int mode, int par)
     {
         hipStream_t st = e.st;
         const bool iter = mode == BMODE_ITER;
+        const Geo& g = iter ? gi() : gs();
         BPtr<T> bp = bptr_t<T>(par);
         Ptr<T> yp = yptr_t<T>(par);
-        bfast::launch_z<T>(beh, iter ? BMODE_ITER : BMODE_START, gf, bp, st, lin);
-        if (mode == BMODE_START) bfin1<BMODE_START>(gf);
+        const int zm = iter ? BMODE_ITER : BMODE_START;
+        if (fast) bfast::launch_z<T>(beh, zm, g, bp, st, lin);
+        else if constexpr (sizeof(T) == 8)
+            bflex::launch_z(beh, zm, g, bp, st, lin);
+        if (mode == BMODE_START) bfin1<BMODE_START>(g);
         else if (mode == BMODE_RESTART)
-            bfin1<BMODE_RESTART>(gf);
-        else bfin1<BMODE_ITER>(gf);
-        if (iter) bfast::launch_y6_fwd<T>(gf6, yp, st);
-        else bfast::launch_y12<T>(gf, yp, st);
-        bfast::launch_x<T>(gf, bp, st, iter);
-        hipLaunchKernelGGL((k_bfin2<0>), dim3(1), dim3(FTHREADS), 0, st, gf, ctl, pchk);
-        bfast::launch_y6<T>(gf6, yp, st);
+            bfin1<BMODE_RESTART>(g);
+        else bfin1<BMODE_ITER>(g);
+        if (fast) {
+            if (iter) bfast::launch_y6_fwd<T>(gf6, yp, st);
+            else bfast::launch_y12<T>(gf, yp, st);
+            bfast::launch_x<T>(gf, bp, st, iter);
+        } else if constexpr (sizeof(T) == 8) {
+            flex::launch_y<T>(-1, BUF_K, 0, g, yp, st);
+            bflex::launch_x(g, bp, st, iter);
+        }
+        hipLaunchKernelGGL((k_bfin2<0>), dim3(1), dim3(FTHREADS), 0, st, g, ctl, pchk);
+        if (fast) bfast::launch_y6<T>(gf6, yp, st);
+        else if constexpr (sizeof(T) == 8)
+            flex::launch_y<T>(1, BUF_MAIN, 0, g6, yp, st);
     }
 
-    // the fields and state of the increment's last iterate on the
-    // specialised FP64 path, whose iterations do not store them: the z pass
+    // the fields and state of the increment's last iterate on the FP64 path,
+    // whose iterations do not store them: the z pass
     // in FINAL mode on the S6 buffer that iterate was computed from (for
     // "ep" it also leaves the export sums in pfin and applies
     // update_old_Variable).  The
@@ -258,13 +241,15 @@ struct BasicRunner {
     // buffer 0, so iterate itNo c.it read buffer (c.it - it0 - 1) & 1.  The
     // z pass skips a solve marked done, so the flag is cleared around it; c
     // is the host copy of the control block after the iterations.
-    void final_fast(Ctl& c, int it0)
+    void finish(Ctl& c, int it0)
     {
         hipStream_t st = e.st;
         Ctl run = c;
         run.done = 0;
         HCHK(hipMemcpyAsync(ctl, &run, sizeof run, hipMemcpyHostToDevice, st));
-        bfast::launch_z<double>(beh, BMODE_FINAL, gf, bptr_t<double>((c.it - it0 - 1) & 1), st, lin);
+        const BPtr<double> bp = bptr_t<double>((c.it - it0 - 1) & 1);
+        if (fast) bfast::launch_z<double>(beh, BMODE_FINAL, gf, bp, st, lin);
+        else bflex::launch_z(beh, BMODE_FINAL, g6, bp, st, lin);
         HCHK(hipGetLastError());
         Ctl after;
         HCHK(hipMemcpyAsync(&after, ctl, sizeof after, hipMemcpyDeviceToHost, st));
@@ -272,13 +257,6 @@ struct BasicRunner {
         if (after.err) c.done = 3;
         HCHK(hipMemcpyAsync(ctl, &c, sizeof c, hipMemcpyHostToDevice, st));
         HCHK(hipStreamSynchronize(st));
-    }
-
-    void run_stage(int mode, int par)
-    {
-        if (fast) stage_fast(mode, par);
-        else if (g12.gen) stage<true>(mode);
-        else stage<false>(mode);
     }
 
     // mtab: per phase {la, mu, Sy, H, n, P, Y0, 0}; la0/mu0: reference medium;
@@ -332,8 +310,8 @@ struct BasicRunner {
         auto capture = [&](GraphGuard& gg, bool fp32) {
             HCHK(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
             for (int k = 0; k < ck; ++k) {
-                if (fp32) stage_fast<float>(BMODE_ITER, k & 1);
-                else run_stage(BMODE_ITER, k & 1);
+                if (fp32) stage<float>(BMODE_ITER, k & 1);
+                else stage(BMODE_ITER, k & 1);
             }
             HCHK(hipStreamEndCapture(st, &gg.g));
             hipError_t ge = hipGraphInstantiate(&gg.x, gg.g, nullptr, nullptr, 0);
@@ -370,7 +348,7 @@ struct BasicRunner {
                 HCHK(hipMemcpyAsync(ctl, &c, sizeof c, hipMemcpyHostToDevice, st));
                 hipLaunchKernelGGL((k_bcopy<double, float>), dim3(nb), dim3(256), 0, st, g12, bp, bp32,
                                    BC_EPS | BC_SIGOLD | BC_EPSOLD | BC_EP);
-                stage_fast<float>(BMODE_START, 1);
+                stage<float>(BMODE_START, 1);
                 HCHK(hipGetLastError());
                 replay(g32.x);
                 if (c.done == 2) {
@@ -391,11 +369,11 @@ struct BasicRunner {
                     c.tol_eq = tol_eq;
                     const int it0 = c.it;
                     HCHK(hipMemcpyAsync(ctl, &c, sizeof c, hipMemcpyHostToDevice, st));
-                    stage_fast<double>(BMODE_RESTART, 1);
+                    stage<double>(BMODE_RESTART, 1);
                     HCHK(hipGetLastError());
                     replay(g64.x);
                     if (c.done != 3) {
-                        final_fast(c, it0);
+                        finish(c, it0);
                         fused = beh == BEH_EP;
                     }
                     fp64_run = false;
@@ -411,11 +389,11 @@ struct BasicRunner {
                 c.tol_f = tol_f;
                 c.tol_eq = tol_eq;
                 HCHK(hipMemcpyAsync(ctl, &c, sizeof c, hipMemcpyHostToDevice, st));
-                run_stage(BMODE_START, 1);
+                stage(BMODE_START, 1);
                 HCHK(hipGetLastError());
                 replay(g64.x);
-                if (fast && c.done != 3) {
-                    final_fast(c, 0);
+                if (c.done != 3) {
+                    finish(c, 0);
                     fused = beh == BEH_EP;
                 }
             }
@@ -430,7 +408,7 @@ struct BasicRunner {
             // export_homogen_var(inc) (:722-746): from the fused FINAL pass's
             // block sums, or from the fields
             if (fused)
-                hipLaunchKernelGGL((k_bfsums<0>), dim3(nblk, 14), dim3(256), 0, st, gf, (const double*)pfin, bs, nblk);
+                hipLaunchKernelGGL((k_bfsums<0>), dim3(nblk, 14), dim3(256), 0, st, gi(), (const double*)pfin, bs, nblk);
             else if (beh == BEH_EP)
                 hipLaunchKernelGGL((k_bsums<double, BEH_EP>), dim3(nblk, 1), dim3(256), 0, st, g12, bp, bs, nblk);
             else
@@ -460,14 +438,14 @@ struct BasicRunner {
                 break;
             }
             // update_old_Variable (:693-719); E += dE does not feed back (updateE recomputes E).
-            // The fused FINAL pass has applied it; else here, and on the specialised
-            // kernels sigma_star for the next start stage
+            // The fused FINAL pass has applied it; else here, with sigma_star for the
+            // next start stage
             if (!fused) {
                 if (beh == BEH_EP)
                     hipLaunchKernelGGL((k_bupdate<double, BEH_EP>), dim3(8192), dim3(256), 0, st, g12, bp, 1);
                 else
                     hipLaunchKernelGGL((k_bupdate<double, BEH_ED>), dim3(8192), dim3(256), 0, st, g12, bp, 1);
-                if (beh == BEH_EP && fast) hipLaunchKernelGGL((k_bstar<double>), dim3(8192), dim3(256), 0, st, g12, bp);
+                if (beh == BEH_EP) hipLaunchKernelGGL((k_bstar<double>), dim3(8192), dim3(256), 0, st, g12, bp);
             }
         }
         HCHK(hipEventRecord(e.ev1, st));

@@ -27,12 +27,11 @@
 #include "../../include/m3d.h"
 #include "m3d_kernels.hpp"
 #include "m3d_fast.hpp"
+#include "m3d_flex.hpp"
 
 using namespace m3d;
 
 namespace {
-
-constexpr size_t LDS_MAX = 65536;
 
 // spectrum layout of the specialised kernels: x planes per block (power of
 // two; 1 = plain [x][y][kz] rows) and, for plain rows, extra complex values
@@ -75,31 +74,6 @@ struct ArgError {
 };
 
 // ------------------------------------------------------------ FFT planning
-bool make_axis(int L, int table_len, FftAxis& a)
-{
-    std::memset(&a, 0, sizeof a);
-    a.L = L;
-    a.tws = table_len / L;
-    int m = L, e2 = 0;
-    while (m % 2 == 0) { m /= 2; ++e2; }
-    std::vector<int> r;
-    // powers of two: radix 8 where possible, 4*4 instead of 8*2
-    while (e2 >= 3) {
-        if (e2 == 4) { r.push_back(4); r.push_back(4); e2 = 0; break; }
-        r.push_back(8);
-        e2 -= 3;
-    }
-    if (e2 == 2) r.push_back(4);
-    if (e2 == 1) r.push_back(2);
-    for (int p : {3, 5, 7, 11, 13})
-        while (m % p == 0) { r.push_back(p); m /= p; }
-    if (m != 1 || (int)r.size() > 16) return false;
-    a.np = (int)r.size();
-    a.rad = 0;
-    for (int i = 0; i < a.np; ++i) a.rad |= (unsigned long long)r[i] << (4 * i);
-    return true;
-}
-
 template <typename T>
 std::vector<cx<T>> twiddles(int n)
 {
@@ -111,38 +85,21 @@ std::vector<cx<T>> twiddles(int n)
     return t;
 }
 
-// tile shapes for precision of complex size csz
-void plan_tiles(Geo& g, size_t csz)
+// line lengths accepted: a line group of C components fits one workgroup's
+// tile in either precision, and no prime factor above 13
+void check_lines(int Nx, int Ny, int Nz, int C)
 {
-    const int C = g.C;
-    const int Lz = g.zeven ? g.Nz / 2 : g.Nz;
-    g.lsz = g.zeven ? g.Nzh : g.Nz;
-    g.TY = 0;
-    for (int ty = g.Ny; ty >= 1; --ty) {
-        if (g.Ny % ty) continue;
-        if ((long)ty * C * Lz > (long)EPT * ZTHREADS) continue;
-        if ((size_t)ty * C * g.lsz * csz > LDS_MAX) continue;
-        g.TY = ty;
-        break;
-    }
-    if (!g.TY) throw ArgError{M3D_ERR_UNSUPPORTED, "z line too long for one workgroup"};
-    g.nty = g.Ny / g.TY;
-    auto tk = [&](int L) {
-        long a = (long)EPT * XYTHREADS / ((long)C * L);
-        long b = (long)(LDS_MAX / ((size_t)C * L * csz));
-        long t = std::min(a, b);
-        t = std::min<long>(t, g.Nzh);
-        return (int)t;
-    };
-    g.TKy = tk(g.Ny);
-    g.TKx = tk(g.Nx);
-    if (g.TKy < 1 || g.TKx < 1) throw ArgError{M3D_ERR_UNSUPPORTED, "x/y line too long for one workgroup"};
-    g.nky = (g.Nzh + g.TKy - 1) / g.TKy;
-    g.nkx = (g.Nzh + g.TKx - 1) / g.TKx;
-    g.nbz = g.Nx * g.nty;
-    g.nbx = g.Ny * g.nkx;
-    g.TKc = g.TKx;
-    g.nbc = g.nbx;
+    const int lsz = Nz % 2 == 0 ? Nz / 2 + 1 : Nz;
+    if ((long)C * lsz > 4096) throw ArgError{M3D_ERR_UNSUPPORTED, "z line too long for one workgroup"};
+    if ((long)C * std::max(Nx, Ny) > 4096) throw ArgError{M3D_ERR_UNSUPPORTED, "x/y line too long for one workgroup"};
+    for (int L : {Nx, Ny, Nz})
+        for (int q : {2, 3, 5, 7, 11, 13, 0}) {
+            if (q == 0) {
+                if (L != 1) throw ArgError{M3D_ERR_UNSUPPORTED, "grid size has a prime factor larger than 13"};
+            } else {
+                while (L % q == 0) L /= q;
+            }
+        }
 }
 
 // line lengths with compile-time specialised kernels (per physics)
@@ -168,16 +125,12 @@ Geo make_geo(int Nx, int Ny, int Nz, int C)
     g.H = (long long)Nx * Ny * g.Nzh;
     g.zeven = (Nz % 2 == 0);
     g.invN = 1.0 / (double)g.N;
-    if (!make_axis(g.zeven ? Nz / 2 : Nz, Nz, g.az) || !make_axis(Ny, Ny, g.ay) || !make_axis(Nx, Nx, g.ax))
-        throw ArgError{M3D_ERR_UNSUPPORTED, "grid size has a prime factor larger than 13"};
-    plan_tiles(g, csz);
-    const FftAxis* a[3] = {&g.az, &g.ay, &g.ax};
-    for (const FftAxis* x : a)
-        for (int i = 0; i < x->np; ++i) {
-            const int r = x->radix(i);
-            if (r != 2 && r != 3 && r != 4 && r != 8) g.gen = 1;
-        }
-    // compile-time specialised passes where available
+    check_lines(Nx, Ny, Nz, C);
+    if (!flex::make_axis(Nz, g.az) || !flex::make_axis(Ny, g.ay) || !flex::make_axis(Nx, g.ax))
+        throw ArgError{M3D_ERR_UNSUPPORTED, "grid size without a radix plan"};
+    flex::plan(g, csz);
+    // compile-time specialised passes where available, the passes of
+    // m3d_flex.hpp along the other axes
     // the z kernels are instantiated for the tile a cubic grid would use
     if (g.zeven && fast_z(C, Nz / 2) && fast::zlines<T>(Nz / 2, C, Ny) == fast::zlines<T>(Nz / 2, C, Nz)) {
         g.fz = 1;
@@ -198,12 +151,11 @@ Geo make_geo(int Nx, int Ny, int Nz, int C)
         g.TKc = fast::xctile<T>(Nx, C);
         g.nbc = Ny * ((g.Nzh + g.TKc - 1) / g.TKc);
     }
-    // spectrum row layout (the runtime-planned kernels address rows (x, y)
-    // at (x * Ny + y) * Nzh * C: plain rows without padding)
+    // spectrum row layout
     const long long rowc = (long long)g.Nzh * C;
     const bool all_fast = g.fz && g.fy && g.fx;
-    // the specialised kernels may start every row on an M3D_ROW_ALIGN-byte
-    // boundary (whole kz slots of padding): their y and x passes move a row's
+    // every row may start on an M3D_ROW_ALIGN-byte boundary (whole kz slots of
+    // padding): the y and x passes move a row's
     // kz tile as one contiguous chunk, and a chunk that straddles 64-byte
     // sectors is written as partial sectors (measured: 64-byte rows made the
     // z and y passes slower).  By default rows are padded to 16 bytes only,
@@ -212,8 +164,7 @@ Geo make_geo(int Nx, int Ny, int Nz, int C)
     // 16-byte pairs too
     long long rowp = rowc;
     constexpr long long row_align = M3D_ROW_ALIGN > 0 ? M3D_ROW_ALIGN : 16;
-    if (all_fast)
-        while ((rowp * (long long)csz) % row_align) rowp += C;
+    while ((rowp * (long long)csz) % row_align) rowp += C;
     g.lxb = 0;
     g.xbm = 0;
     g.sxb = rowp;
@@ -224,7 +175,7 @@ Geo make_geo(int Nx, int Ny, int Nz, int C)
         g.xbm = M3D_XBLOCK - 1;
         g.sxa = (long long)Ny * M3D_XBLOCK * rowp;
         g.sy = (long long)M3D_XBLOCK * rowp;
-    } else if (all_fast) {
+    } else {
         g.sxa += M3D_XPAD; // x planes M3D_XPAD complex values apart beyond their rows
     }
     g.spec = (long long)((Nx - 1) >> g.lxb) * g.sxa + (long long)((Nx - 1) & g.xbm) * g.sxb + (long long)(Ny - 1) * g.sy + rowc;
@@ -648,16 +599,8 @@ struct Engine {
             if (!ok) throw ArgError{M3D_ERR_UNSUPPORTED, "no z kernel"};
             return;
         }
-        const size_t zsm = (size_t)g.TY * C * g.lsz * sizeof(cx<T>);
-        const dim3 grid(g.nsolve * g.nbz);
-        // the generic kernel adds r of anchored solves at run time; the anchor
-        // mode is the specialised kernels' only (callers check g.fz)
         static_assert((MODE != MODE_IUA && MODE != MODE_FWDP) || sizeof(T) == 8, "polish modes are FP64");
-        if (MODE == MODE_IUA || MODE == MODE_FWDP)
-            throw ArgError{M3D_ERR_STATE, "polish z pass without the specialised kernels"};
-        constexpr int GM = (MODE == MODE_IUFR || MODE == MODE_IUA) ? MODE_IUF : (MODE == MODE_FWDP ? MODE_FWD : MODE);
-        if (g.gen) hipLaunchKernelGGL((k_zpass<T, PH, GM, true>), grid, dim3(ZTHREADS), zsm, st, g, p);
-        else hipLaunchKernelGGL((k_zpass<T, PH, GM, false>), grid, dim3(ZTHREADS), zsm, st, g, p);
+        flex::launch_z<T, PH>(MODE, g, p, st);
     }
 
     // threads of a finaliser workgroup over n partial sums per solve: the
@@ -765,10 +708,8 @@ struct Engine {
             if (!xyfast<T, 0, DIR, WHICH>(g, p)) throw ArgError{M3D_ERR_UNSUPPORTED, "no y kernel"};
             return;
         }
-        const size_t ysm = (size_t)g.Ny * g.TKy * C * sizeof(cx<T>);
-        const dim3 grid(g.nsolve * g.Nx * g.nky);
-        if (g.gen) hipLaunchKernelGGL((k_ypass<T, C, DIR, WHICH, true>), grid, dim3(XYTHREADS), ysm, st, g, p);
-        else hipLaunchKernelGGL((k_ypass<T, C, DIR, WHICH, false>), grid, dim3(XYTHREADS), ysm, st, g, p);
+        constexpr unsigned cap = M3D_CHK_WG > 0 ? M3D_CHK_WG : PH::chk_grid;
+        flex::launch_y<T>(DIR, WHICH, cap, g, p, st);
     }
 
     template <typename T>
@@ -778,10 +719,7 @@ struct Engine {
             if (!xyfast<T, 1, -1, BUF_MAIN>(g, p)) throw ArgError{M3D_ERR_UNSUPPORTED, "no x kernel"};
             return;
         }
-        const size_t xsm = (size_t)g.Nx * g.TKx * C * sizeof(cx<T>);
-        const dim3 grid(g.nsolve * g.nbx);
-        if (g.gen) hipLaunchKernelGGL((k_xgreen<T, PH, true>), grid, dim3(XYTHREADS), xsm, st, g, p, prm<T>());
-        else hipLaunchKernelGGL((k_xgreen<T, PH, false>), grid, dim3(XYTHREADS), xsm, st, g, p, prm<T>());
+        flex::launch_xgreen<T, PH>(g, p, prm<T>(), st);
     }
 
     template <typename T, int WHICH>
@@ -791,15 +729,12 @@ struct Engine {
             if (!xyfast<T, 2, -1, WHICH>(g, p)) throw ArgError{M3D_ERR_UNSUPPORTED, "no x check kernel"};
             return;
         }
-        const size_t xsm = (size_t)g.Nx * g.TKx * C * sizeof(cx<T>);
-        const dim3 grid(g.nsolve * g.nbx);
-        if (g.gen) hipLaunchKernelGGL((k_xcheck<T, PH, WHICH, true>), grid, dim3(XYTHREADS), xsm, st, g, p);
-        else hipLaunchKernelGGL((k_xcheck<T, PH, WHICH, false>), grid, dim3(XYTHREADS), xsm, st, g, p);
+        flex::launch_xcheck<T, PH>(WHICH, g, p, st);
     }
 
-    template <typename T>
     // promote: the FP64 start of the polish reads the FP32 iterate and writes
-    // its FP64 copy itself (specialised kernels; k_promote otherwise)
+    // its FP64 copy itself
+    template <typename T>
     void launch_start(const Geo& g, const Ptr<T>& p, bool promote = false)
     {
         if constexpr (sizeof(T) == 8) {
@@ -820,10 +755,9 @@ struct Engine {
     template <typename T>
     void launch_iter(const Geo& g, const Ptr<T>& p, bool green = true)
     {
-        // the FP64 anchor iteration on the specialised kernels also writes r
-        // and e (MODE_IUA; k_anchor otherwise)
+        // the FP64 anchor iteration also writes r and e (MODE_IUA)
         if constexpr (sizeof(T) == 8) {
-            if (!green && g.fz) zpass<T, MODE_IUA>(g, p);
+            if (!green) zpass<T, MODE_IUA>(g, p);
             else zpass<T, MODE_IUF>(g, p);
         } else {
             zpass<T, MODE_IUF>(g, p);
@@ -923,14 +857,13 @@ struct Engine {
         run_graph(chunk_for(g), [&]() { launch_iter<T>(g, p); }, hctl);
     }
 
-    // anchored polish of the solves flagged corr (r and e from k_anchor, or
-    // from the anchor iteration's z pass on the specialised kernels)
+    // anchored polish of the solves flagged corr (r and e from the anchor
+    // iteration's z pass)
     void run_corr(Geo gf, Geo gd, std::vector<Ctl>& hctl)
     {
         gf.nsolve = gd.nsolve = nsolve;
         Ptr<float> pf = ptrs<float>(gf);
         Ptr<double> pd = ptrs<double>(gd);
-        if (!gd.fz) hipLaunchKernelGGL((k_anchor<C>), dim3(1024), dim3(256), 0, st, gd, pd, pf, ctl);
         launch_start_corr(gf, pf);
         HCHK(hipGetLastError());
         run_graph(chunk_for(gf), [&]() { launch_iter_corr(gf, pf, gd, pd); }, hctl);
@@ -1124,10 +1057,9 @@ struct Engine {
                 hctl[s].tol_eq = tol_eq;
             }
             HCHK(hipMemcpyAsync(ctl, hctl.data(), sizeof(Ctl) * nsolve, hipMemcpyHostToDevice, st));
-            // promote the FP32 iterates to FP64: inside the polish's first z pass
-            // on the specialised kernels, else by k_promote
-            const bool fused_promote = refine && gd.fz;
-            if (!fused_promote)
+            // promote the FP32 iterates to FP64: inside the polish's first z pass,
+            // or by k_promote for plain FP64 polish iterations
+            if (!refine)
                 hipLaunchKernelGGL((k_promote<C>), dim3(1024), dim3(256), 0, st, gd, ptrs<float>(gf), ptrs<double>(gd), ctl);
             bool any = false;
             for (int s = 0; s < nsolve; ++s) any = any || (hctl[s].done == 0);
@@ -1138,7 +1070,7 @@ struct Engine {
                 // taken in FP64 from A + e.  The corrections transform e only,
                 // so that iteration stops after its update and stop check.
                 Ptr<double> pd = ptrs<double>(gd);
-                launch_start<double>(gd, pd, fused_promote);
+                launch_start<double>(gd, pd, true);
                 launch_iter<double>(gd, pd, false);
                 HCHK(hipGetLastError());
                 HCHK(hipMemcpyAsync(hctl.data(), ctl, sizeof(Ctl) * nsolve, hipMemcpyDeviceToHost, st));

@@ -292,7 +292,7 @@ __device__ __forceinline__ void pass(cx<T>* __restrict__ s, const cx<T>* __restr
                 if (Ns > 1 && r > 0) a = twmul<DIR>(a, tw[k * r * tstep]);
                 v[i][r] = a;
             }
-            butterfly<T, R, DIR>(v[i], tw, 0);
+            butterfly<T, R, DIR>(v[i]);
         }
     }
     __syncthreads();

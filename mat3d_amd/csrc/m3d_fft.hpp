@@ -1,18 +1,13 @@
-// m3d_fft.hpp -- LDS-resident Stockham FFT building blocks for gfx950.
+// m3d_fft.hpp -- complex arithmetic and the in-register butterflies of the
+// LDS-resident Stockham FFTs (gfx950).
 //
 // A workgroup owns a tile of lines in LDS and transforms all of them with a
 // sequence of in-place Stockham passes: every thread loads the R inputs of
-// each of its butterflies into registers, the workgroup synchronises, the
-// butterflies are computed and stored to their autosorted positions.  No
-// bit reversal pass is needed and the output is in natural order.
-//
-// Lines are described by a two-level geometry so one routine covers both
-// layouts used by the solver:
-//   * "interleaved" lines (y/x passes): element e of line l lives at
-//     l + e*es (es = number of lines), consecutive threads take consecutive
-//     lines -> conflict-free LDS access;
-//   * "contiguous" lines (z pass): element e of line l at l*ls + e,
-//     consecutive threads take consecutive elements.
+// each of its butterflies into registers, the butterflies are computed, the
+// workgroup synchronises and stores them to their autosorted positions.  No
+// bit reversal pass is needed and the output is in natural order.  The
+// passes themselves are in m3d_fast.hpp (compile-time line lengths) and
+// m3d_flex.hpp (any product of primes up to 13).
 //
 // Twiddles come from a per-axis table tw[m] = exp(-2 pi i m / Ltab); a pass
 // over lines of length L uses stride Ltab/L into it.
@@ -48,18 +43,104 @@ __device__ __forceinline__ cx<T> rot90(cx<T> a)
     return DIR < 0 ? cx<T>{a.im, -a.re} : cx<T>{-a.im, a.re};
 }
 
+// radix sequence of one axis' line FFT
 struct FftAxis {
     int L;                   // transform length
     int np;                  // number of passes (<= 16)
-    int tws;                 // stride into the twiddle table (table length / L)
-    int pad;
-    unsigned long long rad;  // radix of pass p in bits [4p, 4p+4) (kept packed so the
+    unsigned long long rad;  // radix - 1 of pass p in bits [4p, 4p+4) (kept packed so the
                              // kernel never indexes its by-value arguments dynamically)
-    __host__ __device__ int radix(int p) const { return (int)((rad >> (4 * p)) & 15ull); }
+    __host__ __device__ int radix(int p) const { return (int)((rad >> (4 * p)) & 15ull) + 1; }
+};
+
+// cos and sin of 2 pi p / q as compile-time constants: the angle is reduced
+// to [0, pi/4] in exact integer arithmetic and carried as x + lo (Dekker's
+// product gives the rounding of x), then summed by its Taylor series from the
+// smallest term
+constexpr double root_series(long long p, long long q, bool cosine)
+{
+    const double pi2 = 2 * 3.14159265358979323846, pi2_lo = 2 * 1.2246467991473532e-16;
+    const double x = pi2 * (double)p / (double)q;
+    auto split = [](double a, double& h, double& l) {
+        const double c = 134217729.0 * a; // 2^27 + 1
+        h = c - (c - a);
+        l = a - h;
+    };
+    auto prod_err = [&](double a, double b) { // a b - fl(a b)
+        double ah = 0, al = 0, bh = 0, bl = 0;
+        split(a, ah, al);
+        split(b, bh, bl);
+        return ((ah * bh - a * b) + ah * bl + al * bh) + al * bl;
+    };
+    const double num = pi2 * (double)p, back = x * (double)q;
+    const double lo = ((num - back) + (prod_err(pi2, (double)p) - prod_err(x, (double)q)) + pi2_lo * (double)p) / (double)q;
+    double c = 0, s = 0; // cos x - 1 and (sin x - x) by Horner's rule
+    for (int i = 26; i >= 2; i -= 2) {
+        c = -x * x / (double)((i - 1) * i) * (1.0 + c);
+        s = -x * x / (double)(i * (i + 1)) * (1.0 + s);
+    }
+    return cosine ? 1.0 + (c - lo * x) : x + (x * s + lo * (1.0 + c));
+}
+constexpr double root_sin(long long p, long long q);
+constexpr double root_cos(long long p, long long q)
+{
+    p %= q;
+    if (p < 0) p += q;
+    if (2 * p > q) p = q - p;                                   // cos(2 pi - a) = cos a
+    if (4 * p > q) return -root_cos(q - 2 * p, 2 * q);          // cos(pi - a) = -cos a
+    if (8 * p > q) return root_series(q - 4 * p, 4 * q, false); // cos a = sin(pi/2 - a)
+    return root_series(p, q, true);
+}
+constexpr double root_sin(long long p, long long q) { return root_cos(4 * p - q, 4 * q); } // cos(a - pi/2)
+template <int N>
+struct RootTab {
+    double c[N] = {}, s[N] = {}; // of 2 pi m / N
+    constexpr RootTab()
+    {
+        for (int m = 0; m < N; ++m) {
+            c[m] = root_cos(m, N);
+            s[m] = root_sin(m, N);
+        }
+    }
 };
 
 template <typename T, int R, int DIR>
-__device__ __forceinline__ void butterfly(cx<T> (&v)[R], const cx<T>* __restrict__ tw, int wstep)
+__device__ __forceinline__ void butterfly(cx<T> (&v)[R]);
+
+// R = A B points: A-point DFTs over n1 of v[B n1 + n2], twiddles W_R^(n2 k1),
+// B-point DFTs over n2; X[k1 + A k2] lands in v[k1 + A k2]
+template <typename T, int A, int B, int DIR>
+__device__ __forceinline__ void butterfly_ab(cx<T> (&v)[A * B])
+{
+    constexpr RootTab<A * B> rt;
+    cx<T> y[B][A];
+#pragma unroll
+    for (int n2 = 0; n2 < B; ++n2) {
+        cx<T> t[A];
+#pragma unroll
+        for (int n1 = 0; n1 < A; ++n1) t[n1] = v[B * n1 + n2];
+        butterfly<T, A, DIR>(t);
+#pragma unroll
+        for (int k1 = 0; k1 < A; ++k1) {
+            if (n2 * k1 == 0) y[n2][k1] = t[k1];
+            else {
+                const T c = T(rt.c[n2 * k1]), s = T(DIR > 0 ? rt.s[n2 * k1] : -rt.s[n2 * k1]);
+                y[n2][k1] = cx<T>{t[k1].re * c - t[k1].im * s, t[k1].re * s + t[k1].im * c};
+            }
+        }
+    }
+#pragma unroll
+    for (int k1 = 0; k1 < A; ++k1) {
+        cx<T> u[B];
+#pragma unroll
+        for (int n2 = 0; n2 < B; ++n2) u[n2] = y[n2][k1];
+        butterfly<T, B, DIR>(u);
+#pragma unroll
+        for (int k2 = 0; k2 < B; ++k2) v[k1 + A * k2] = u[k2];
+    }
+}
+
+template <typename T, int R, int DIR>
+__device__ __forceinline__ void butterfly(cx<T> (&v)[R])
 {
     if constexpr (R == 2) {
         cx<T> a = v[0], b = v[1];
@@ -150,108 +231,47 @@ __device__ __forceinline__ void butterfly(cx<T> (&v)[R], const cx<T>* __restrict
             v[k1 + 8] = s02 - s13;
             v[k1 + 12] = d02 - d13;
         }
+    } else if constexpr (R == 6) {
+        butterfly_ab<T, 3, 2, DIR>(v);
+    } else if constexpr (R == 9) {
+        butterfly_ab<T, 3, 3, DIR>(v);
+    } else if constexpr (R == 10) {
+        butterfly_ab<T, 5, 2, DIR>(v);
+    } else if constexpr (R == 12) {
+        butterfly_ab<T, 3, 4, DIR>(v);
+    } else if constexpr (R == 14) {
+        butterfly_ab<T, 7, 2, DIR>(v);
+    } else if constexpr (R == 15) {
+        butterfly_ab<T, 5, 3, DIR>(v);
     } else {
-        // generic odd radix: direct DFT, W_R^m = tw[m * wstep]
-        cx<T> out[R];
+        // odd prime: sums and differences of the pairs (m, R - m), then
+        //   X_q, X_(R-q) = A_q -/+ i B_q,  A_q = v0 + sum_m cos(2 pi q m / R) (v_m + v_(R-m)),
+        //   B_q = sum_m sin(2 pi q m / R) (v_m - v_(R-m))     (signs for the forward transform)
+        static_assert(R == 5 || R == 7 || R == 11 || R == 13, "radix");
+        constexpr int H = (R - 1) / 2;
+        constexpr RootTab<R> rt;
+        cx<T> t[H], d[H];
+        cx<T> x0 = v[0];
 #pragma unroll
-        for (int q = 0; q < R; ++q) {
-            cx<T> acc = v[0];
+        for (int m = 1; m <= H; ++m) {
+            t[m - 1] = v[m] + v[R - m];
+            d[m - 1] = v[m] - v[R - m];
+            x0 = x0 + t[m - 1];
+        }
 #pragma unroll
-            for (int r = 1; r < R; ++r) {
-                cx<T> w = tw[((r * q) % R) * wstep];
-                if (DIR > 0) w.im = -w.im;
-                acc = acc + cmul(v[r], w);
+        for (int q = 1; q <= H; ++q) {
+            cx<T> a = v[0], b{T(0), T(0)};
+#pragma unroll
+            for (int m = 1; m <= H; ++m) {
+                const T c = T(rt.c[q * m % R]), s = T(rt.s[q * m % R]);
+                a = cx<T>{a.re + c * t[m - 1].re, a.im + c * t[m - 1].im};
+                b = cx<T>{b.re + s * d[m - 1].re, b.im + s * d[m - 1].im};
             }
-            out[q] = acc;
+            b = rot90<DIR>(b);
+            v[q] = a + b;
+            v[R - q] = a - b;
         }
-#pragma unroll
-        for (int q = 0; q < R; ++q) v[q] = out[q];
-    }
-}
-
-// Line geometry inside LDS: offset(l) = (l % nin)*lin + (l / nin)*lout,
-// element stride es.
-struct LineGeo {
-    int nl;   // number of lines
-    int nin;  // lines in the inner group
-    int lin;  // stride between inner lines
-    int lout; // stride between inner groups
-    int es;   // element stride
-    __device__ __forceinline__ int off(int l) const { return (l % nin) * lin + (l / nin) * lout; }
-};
-
-// One in-place Stockham pass of radix R over all lines of the tile.
-// EPT bounds the number of complex values a thread holds (items*R).
-template <typename T, int R, int DIR, int EPT, bool LINES_FAST>
-__device__ __forceinline__ void fft_pass(cx<T>* __restrict__ s, const LineGeo g, int L, int Ns,
-                                         const cx<T>* __restrict__ tw, int tws)
-{
-    constexpr int IPT = (EPT + R - 1) / R;
-    const int nR = L / R;
-    const int items = g.nl * nR;
-    const int tstep = (L / (Ns * R)) * tws;
-    const int nthr = blockDim.x;
-    cx<T> v[IPT][R];
-#pragma unroll
-    for (int i = 0; i < IPT; ++i) {
-        const int it = threadIdx.x + i * nthr;
-        if (it < items) {
-            int l, j;
-            if (LINES_FAST) { l = it % g.nl; j = it / g.nl; }
-            else { j = it % nR; l = it / nR; }
-            const int lo = g.off(l);
-            const int k = j % Ns;
-#pragma unroll
-            for (int r = 0; r < R; ++r) {
-                cx<T> a = s[lo + (j + r * nR) * g.es];
-                if (r > 0 && Ns > 1) {
-                    cx<T> w = tw[k * r * tstep];
-                    if (DIR > 0) w.im = -w.im;
-                    a = cmul(a, w);
-                }
-                v[i][r] = a;
-            }
-            butterfly<T, R, DIR>(v[i], tw, nR * tws);
-        }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int i = 0; i < IPT; ++i) {
-        const int it = threadIdx.x + i * nthr;
-        if (it < items) {
-            int l, j;
-            if (LINES_FAST) { l = it % g.nl; j = it / g.nl; }
-            else { j = it % nR; l = it / nR; }
-            const int lo = g.off(l);
-            const int k = j % Ns;
-            const int ob = (j / Ns) * Ns * R + k;
-#pragma unroll
-            for (int r = 0; r < R; ++r) s[lo + (ob + r * Ns) * g.es] = v[i][r];
-        }
-    }
-    __syncthreads();
-}
-
-// Full transform of all tile lines (in place).  Radices 2,3,4,8 always;
-// GEN adds the odd radices 5,7,11,13 (kept out of the common instantiation
-// because their register footprint would cap the occupancy of every kernel).
-template <typename T, int DIR, int EPT, bool LINES_FAST, bool GEN>
-__device__ void fft_lines(cx<T>* __restrict__ s, const LineGeo g, const FftAxis ax, const cx<T>* __restrict__ tw)
-{
-    int Ns = 1;
-    for (int p = 0; p < ax.np; ++p) {
-        const int R = ax.radix(p);
-        if (R == 8) fft_pass<T, 8, DIR, EPT, LINES_FAST>(s, g, ax.L, Ns, tw, ax.tws);
-        else if (R == 4) fft_pass<T, 4, DIR, EPT, LINES_FAST>(s, g, ax.L, Ns, tw, ax.tws);
-        else if (R == 3) fft_pass<T, 3, DIR, EPT, LINES_FAST>(s, g, ax.L, Ns, tw, ax.tws);
-        else if (R == 2) fft_pass<T, 2, DIR, EPT, LINES_FAST>(s, g, ax.L, Ns, tw, ax.tws);
-        else if constexpr (GEN) {
-            if (R == 5) fft_pass<T, 5, DIR, EPT, LINES_FAST>(s, g, ax.L, Ns, tw, ax.tws);
-            else if (R == 7) fft_pass<T, 7, DIR, EPT, LINES_FAST>(s, g, ax.L, Ns, tw, ax.tws);
-            else if (R == 11) fft_pass<T, 11, DIR, EPT, LINES_FAST>(s, g, ax.L, Ns, tw, ax.tws);
-            else if (R == 13) fft_pass<T, 13, DIR, EPT, LINES_FAST>(s, g, ax.L, Ns, tw, ax.tws);
-        }
-        Ns *= R;
+        v[0] = x0;
     }
 }
 

@@ -32,17 +32,13 @@
 namespace m3d {
 
 constexpr int NCOEF = 8; // per-phase coefficients
-constexpr int ZTHREADS = 256;
-constexpr int XYTHREADS = 512;
-constexpr int EPT = 16;  // complex values per thread per pass
 
 // z-pass modes: forward only, update (inverse, update, forward), check FFT of
 // the current / previous iterate, update of an anchored FP32 correction (adds
 // r), the FP64 anchor iteration of the polish (inverse and update only;
 // writes r = u_new - u_old and the first correction e = r in FP32), and the
 // FP64 start of the polish from the FP32 iterate (forward only; reads the
-// FP32 ring, writes the promoted FP64 iterate).  The last two: the
-// specialised z pass only.
+// FP32 ring, writes the promoted FP64 iterate).
 enum { MODE_FWD = 0, MODE_IUF = 1, MODE_CHK_CUR = 2, MODE_CHK_PREV = 3, MODE_IUFR = 4, MODE_IUA = 5, MODE_FWDP = 6 };
 enum { BUF_MAIN = 0, BUF_CHK_CUR = 2, BUF_CHK_PREV = 3, BUF_K = 4 };
 
@@ -82,17 +78,16 @@ struct Ctl {
 struct Geo {
     int Nx, Ny, Nz, Nzh, C;
     long long N, H;
-    FftAxis az, ay, ax; // az: Nz/2 (even Nz) or Nz (odd Nz)
+    FftAxis az, ay, ax; // radix plans of the run-time-length passes (m3d_flex.hpp)
     int zeven;
     int TY, nty;        // z tiles: TY lines (y) per tile, Ny/TY tiles per x plane
     int TKy, nky;       // y tiles: TKy kz values, ceil(Nzh/TKy) tiles
     int TKx, nkx;       // x tiles
-    int lsz;            // complex stride of one z line in LDS
     int nsolve;
     int nbz, nbx;       // blocks per solve of the z pass and the x pass
     int TKc, nbc;       // x pass of the equilibrium check: kz tile, partial sums per solve
     double invN;
-    // spectrum layout of the specialised kernels: the half-spectrum row
+    // spectrum layout: the half-spectrum row
     // (x, y) (Nzh*C complex values) starts at
     //   (x >> lxb) * sxa + (x & xbm) * sxb + y * sy
     // plain rows: lxb = 0, xbm = 0, sxa = Ny*Nzh*C (+ padding), sy = Nzh*C;
@@ -101,7 +96,6 @@ struct Geo {
     long long sxa, sxb, sy;
     long long spec;     // complex values of one solve's spectrum (rows + padding)
     int fz, fy, fx;     // host only: compile-time specialised kernel used for this axis
-    int gen;            // host only: generic kernels need the odd radices
 };
 
 template <typename T>
@@ -358,264 +352,6 @@ __device__ __forceinline__ const float* e_buf(const Ptr<T>& p, int it, int s)
     return p.eU + (long long)b * p.eB + (long long)s * p.sU;
 }
 
-// --------------------------------------------------------------- z pass
-// One block: solve s, plane x, lines y0..y0+TY-1, all components.
-// LDS: TY*C lines of lsz complex each; line l = yl*C + c.
-template <typename T, typename PH, int MODE, bool GEN>
-__global__ void __launch_bounds__(ZTHREADS) k_zpass(Geo g, Ptr<T> p)
-{
-    extern __shared__ __align__(16) unsigned char smem_raw[];
-    __shared__ double red[ZTHREADS / 64];
-    constexpr int C = PH::C;
-    cx<T>* sl = reinterpret_cast<cx<T>*>(smem_raw);
-    T* sr = reinterpret_cast<T*>(smem_raw);
-
-    const int per = g.Nx * g.nty;
-    const int s = blockIdx.x / per;
-    const int t = blockIdx.x % per;
-    const int x = t / g.nty;
-    const int y0 = (t % g.nty) * g.TY;
-    const Ctl& ctl = p.ctl[s];
-    if (ctl.done) return;
-    if (MODE == MODE_CHK_CUR && !ctl.need_cur) return;
-    if (MODE == MODE_CHK_PREV && !ctl.need_prev) return;
-    const int it = ctl.it;
-
-    const int Nz = g.Nz, Nzh = g.Nzh, lsz = g.lsz, TY = g.TY;
-    const int nl = TY * C;
-    const long long vox0 = ((long long)x * g.Ny + y0) * Nz;         // first voxel of tile
-    const long long spec0 = ((long long)x * g.Ny + y0) * Nzh * C;  // first spectrum entry
-    const int rv = p.rve_of[s];
-    const uint8_t* ph = p.ph + (long long)rv * p.sPh + vox0;
-    const T* coef = p.coef + (long long)rv * p.sCoef;
-
-    const T* Uin;
-    T* Uout = nullptr;
-    if (MODE == MODE_FWD) Uin = u_buf(p, it, s);
-    else if (MODE == MODE_IUF) { Uin = u_buf(p, it, s); Uout = u_buf(p, it + 1, s); }
-    else if (MODE == MODE_CHK_CUR) Uin = u_buf(p, it, s);
-    else Uin = u_buf(p, it - 1, s);
-    // anchored polish: FP32 updates add r, FP64 checks read anchor + e
-    const bool corr = ctl.corr != 0;
-    const float* Rin = nullptr;
-    const float* Ein = nullptr;
-    if (corr) {
-        if (sizeof(T) == 4 && MODE == MODE_IUF) Rin = p.R + (long long)s * p.sU + vox0 * C;
-        if (sizeof(T) == 8 && (MODE == MODE_CHK_CUR || MODE == MODE_CHK_PREV)) {
-            Uin = u_buf(p, ctl.anc_it, s);
-            Ein = e_buf(p, MODE == MODE_CHK_CUR ? it : it - 1, s) + vox0 * C;
-        }
-    }
-    Uin += vox0 * C;
-    if (Uout) Uout += vox0 * C;
-
-    const LineGeo lg{nl, nl, lsz, 0, 1};
-    const int tid = threadIdx.x, nthr = blockDim.x;
-
-    if (MODE == MODE_IUF) {
-        // 1. load the Green output tile (contiguous in global memory)
-        const cx<T>* src = p.S + (long long)s * p.sS + spec0;
-        const int tot = TY * Nzh * C;
-        for (int e = tid; e < tot; e += nthr) {
-            const int yl = e / (Nzh * C);
-            const int r = e - yl * Nzh * C;
-            const int kz = r / C, c = r - kz * C;
-            sl[(yl * C + c) * lsz + kz] = src[e];
-        }
-        __syncthreads();
-        // 2. c2r pre-processing (real parts of the kz=0 and Nyquist bins only)
-        if (g.zeven) {
-            const int L = Nz / 2;
-            const int half = L / 2 + 1;
-            for (int e = tid; e < nl * half; e += nthr) {
-                const int l = e / half, k = e - l * half;
-                cx<T>* ln = sl + l * lsz;
-                if (k == 0) {
-                    const T x0 = ln[0].re, xl = ln[L].re;
-                    ln[0] = cx<T>{x0 + xl, x0 - xl};
-                } else {
-                    const int kk = L - k;
-                    const cx<T> Xk = ln[k], Xc = ln[kk];
-                    // Z[k]  = (X[k]  + X[kk]*) + i W^-k  (X[k]  - X[kk]*)
-                    // Z[kk] = (X[kk] + X[k]*)  + i W^-kk (X[kk] - X[k]*)
-                    cx<T> w = p.twz[k];
-                    w.im = -w.im;
-                    const cx<T> sm = Xk + cconj(Xc), df = Xk - cconj(Xc);
-                    const cx<T> zk = sm + rot90<1>(cmul(w, df));
-                    ln[k] = zk;
-                    if (kk != k) {
-                        cx<T> w2 = p.twz[kk];
-                        w2.im = -w2.im;
-                        const cx<T> sm2 = Xc + cconj(Xk), df2 = Xc - cconj(Xk);
-                        ln[kk] = sm2 + rot90<1>(cmul(w2, df2));
-                    }
-                }
-            }
-            __syncthreads();
-            fft_lines<T, 1, EPT, false, GEN>(sl, lg, g.az, p.twz);
-        } else {
-            // odd Nz: Hermitian extension, then a full complex inverse FFT
-            for (int e = tid; e < nl * Nzh; e += nthr) {
-                const int l = e / Nzh, k = e - l * Nzh;
-                cx<T>* ln = sl + l * lsz;
-                if (k == 0) ln[0].im = T(0);
-                else ln[Nz - k] = cconj(ln[k]);
-            }
-            __syncthreads();
-            fft_lines<T, 1, EPT, false, GEN>(sl, lg, g.az, p.twz);
-            // pack real parts as reals at the front of the line
-            // (in-place compaction needs a barrier between read and write)
-            T vals[EPT];
-#pragma unroll
-            for (int i = 0; i < EPT; ++i) {
-                const int e = tid + i * nthr;
-                if (e < nl * Nz) vals[i] = sl[(e / Nz) * lsz + (e % Nz)].re;
-            }
-            __syncthreads();
-#pragma unroll
-            for (int i = 0; i < EPT; ++i) {
-                const int e = tid + i * nthr;
-                if (e < nl * Nz) sr[(e / Nz) * 2 * lsz + (e % Nz)] = vals[i];
-            }
-            __syncthreads();
-        }
-    }
-
-    // 3. per-voxel work
-    double acc = 0.0;
-    const int nv = TY * Nz;
-    for (int v = tid; v < nv; v += nthr) {
-        const int yl = v / Nz, z = v - yl * Nz;
-        const T* kp = coef + (int)ph[v] * NCOEF;
-        T u[C], o[C];
-#pragma unroll
-        for (int c = 0; c < C; ++c) u[c] = Uin[(long long)v * C + c];
-        if (Ein) {
-#pragma unroll
-            for (int c = 0; c < C; ++c) u[c] += (T)Ein[(long long)v * C + c];
-        }
-        if (MODE == MODE_IUF) {
-            T d[C], a[C];
-#pragma unroll
-            for (int c = 0; c < C; ++c) d[c] = sr[(yl * C + c) * 2 * lsz + z] - u[c];
-            PH::accel(kp, d, a);
-#pragma unroll
-            for (int c = 0; c < C; ++c) u[c] = u[c] + a[c];
-            if (Rin) {
-#pragma unroll
-                for (int c = 0; c < C; ++c) u[c] += (T)Rin[(long long)v * C + c];
-            }
-#pragma unroll
-            for (int c = 0; c < C; ++c) Uout[(long long)v * C + c] = u[c];
-        }
-        if (MODE == MODE_FWD || MODE == MODE_IUF) {
-            PH::dual(kp, u, o);
-#pragma unroll
-            for (int c = 0; c < C; ++c) acc += (double)o[c];
-            PH::polar(kp, u, o);
-        } else {
-            // sigma: the dual field in the strain (gradient) base, u itself otherwise
-            if (ctl.sb) PH::dual(kp, u, o);
-            else {
-#pragma unroll
-                for (int c = 0; c < C; ++c) o[c] = u[c];
-            }
-        }
-#pragma unroll
-        for (int c = 0; c < C; ++c) sr[(yl * C + c) * 2 * lsz + z] = o[c];
-    }
-    if (MODE == MODE_FWD || MODE == MODE_IUF) {
-        const double bs = block_sum(acc, red);
-        if (tid == 0) p.psum[(long long)s * g.nbz + t] = bs;
-    }
-    __syncthreads();
-
-    // 4. forward r2c along z
-    if (g.zeven) {
-        fft_lines<T, -1, EPT, false, GEN>(sl, lg, g.az, p.twz);
-        const int L = Nz / 2;
-        const int half = L / 2 + 1;
-        for (int e = tid; e < nl * half; e += nthr) {
-            const int l = e / half, k = e - l * half;
-            cx<T>* ln = sl + l * lsz;
-            if (k == 0) {
-                const cx<T> z0 = ln[0];
-                ln[0] = cx<T>{z0.re + z0.im, T(0)};
-                ln[L] = cx<T>{z0.re - z0.im, T(0)};
-            } else {
-                const int kk = L - k;
-                const cx<T> zk = ln[k], zc = cconj(ln[kk]);
-                const cx<T> E = cscale(zk + zc, T(0.5));
-                const cx<T> O = cscale(rot90<-1>(zk - zc), T(0.5)); // -i/2 (zk - zc)
-                ln[k] = E + cmul(p.twz[k], O);
-                if (kk != k) ln[kk] = cconj(E) + cmul(p.twz[kk], cconj(O));
-            }
-        }
-        __syncthreads();
-    } else {
-        // odd Nz: spread reals into complex slots (backwards-safe via registers)
-        T vals[EPT];
-#pragma unroll
-        for (int i = 0; i < EPT; ++i) {
-            const int e = tid + i * nthr;
-            if (e < nl * Nz) vals[i] = sr[(e / Nz) * 2 * lsz + (e % Nz)];
-        }
-        __syncthreads();
-#pragma unroll
-        for (int i = 0; i < EPT; ++i) {
-            const int e = tid + i * nthr;
-            if (e < nl * Nz) sl[(e / Nz) * lsz + (e % Nz)] = cx<T>{vals[i], T(0)};
-        }
-        __syncthreads();
-        fft_lines<T, -1, EPT, false, GEN>(sl, lg, g.az, p.twz);
-    }
-
-    // 5. store the tile (contiguous)
-    {
-        cx<T>* dst = ((MODE == MODE_FWD || MODE == MODE_IUF) ? p.S : p.K) + (long long)s * p.sS + spec0;
-        const int tot = TY * Nzh * C;
-        for (int e = tid; e < tot; e += nthr) {
-            const int yl = e / (Nzh * C);
-            const int r = e - yl * Nzh * C;
-            const int kz = r / C, c = r - kz * C;
-            dst[e] = sl[(yl * C + c) * lsz + kz];
-        }
-    }
-}
-
-// --------------------------------------------------------------- y pass
-// Block: solve s, plane x, kz tile [kz0, kz0+nk); LDS [y][kzl*C + c].
-template <typename T, int C, int DIR, int WHICH, bool GEN>
-__global__ void __launch_bounds__(XYTHREADS) k_ypass(Geo g, Ptr<T> p)
-{
-    extern __shared__ __align__(16) unsigned char smem_raw[];
-    cx<T>* sl = reinterpret_cast<cx<T>*>(smem_raw);
-    const int per = g.Nx * g.nky;
-    const int s = blockIdx.x / per;
-    const int t = blockIdx.x % per;
-    const int x = t / g.nky;
-    const int kz0 = (t % g.nky) * g.TKy;
-    const Ctl& ctl = p.ctl[s];
-    if (ctl.done) return;
-    if (WHICH == BUF_CHK_CUR && !ctl.need_cur) return;
-    if (WHICH == BUF_CHK_PREV && !ctl.need_prev) return;
-    const int nk = min(g.TKy, g.Nzh - kz0);
-    const int w = nk * C;
-    cx<T>* base = (WHICH == BUF_MAIN ? p.S : p.K) + (long long)s * p.sS + ((long long)x * g.Ny * g.Nzh + kz0) * C;
-    const long long ystride = (long long)g.Nzh * C;
-    const int tot = g.Ny * w;
-    for (int e = threadIdx.x; e < tot; e += blockDim.x) {
-        const int y = e / w, r = e - y * w;
-        sl[e] = base[y * ystride + r];
-    }
-    __syncthreads();
-    fft_lines<T, DIR, EPT, true, GEN>(sl, LineGeo{w, w, 1, 0, w}, g.ay, p.twy);
-    for (int e = threadIdx.x; e < tot; e += blockDim.x) {
-        const int y = e / w, r = e - y * w;
-        base[y * ystride + r] = sl[e];
-    }
-}
-
 // ------------------------------------------------ x pass with Green step
 // frequency vector (tensor order z, y, x) of spectrum index (kx, ky, kz)
 __device__ __forceinline__ void freq_el(const Geo& g, int kx, int ky, int kz, int f[3])
@@ -683,111 +419,34 @@ __device__ __forceinline__ void green_apply(const Geo& g, int sb, const T* prm, 
     green_apply_k<T, PH>(g, sb, green_k_of<T, PH::C>(prm), kx, ky, kz, v);
 }
 
-// prm: elastic {la0, mu0}; thermal {k0}
-template <typename T, typename PH, bool GEN>
-__global__ void __launch_bounds__(XYTHREADS) k_xgreen(Geo g, Ptr<T> p, const T* __restrict__ prm_all)
-{
-    extern __shared__ __align__(16) unsigned char smem_raw[];
-    cx<T>* sl = reinterpret_cast<cx<T>*>(smem_raw);
-    constexpr int C = PH::C;
-    const int per = g.Ny * g.nkx;
-    const int s = blockIdx.x / per;
-    const int t = blockIdx.x % per;
-    const int y = t / g.nkx;
-    const int kz0 = (t % g.nkx) * g.TKx;
-    const Ctl& ctl = p.ctl[s];
-    if (ctl.done) return;
-    const T* prm = prm_all + 2 * p.rve_of[s];
-    const int nk = min(g.TKx, g.Nzh - kz0);
-    const int w = nk * C;
-    cx<T>* base = p.S + (long long)s * p.sS + ((long long)y * g.Nzh + kz0) * C;
-    const long long xstride = (long long)g.Ny * g.Nzh * C;
-    const int tot = g.Nx * w;
-    for (int e = threadIdx.x; e < tot; e += blockDim.x) {
-        const int x = e / w, r = e - x * w;
-        sl[e] = base[x * xstride + r];
-    }
-    __syncthreads();
-    const LineGeo lg{w, w, 1, 0, w};
-    fft_lines<T, -1, EPT, true, GEN>(sl, lg, g.ax, p.twx);
-    for (int f = threadIdx.x; f < g.Nx * nk; f += blockDim.x) {
-        const int kx = f / nk, kzl = f - kx * nk;
-        const int kz = kz0 + kzl;
-        cx<T>* v = sl + kx * w + kzl * C;
-        if (kx == 0 && y == 0 && kz == 0) {
-#pragma unroll
-            for (int c = 0; c < C; ++c) v[c] = cx<T>{T(ctl.E[c]), T(0)};
-        } else {
-            green_apply<T, PH>(g, ctl.sb, prm, kx, y, kz, v);
-        }
-    }
-    __syncthreads();
-    fft_lines<T, 1, EPT, true, GEN>(sl, lg, g.ax, p.twx);
-    for (int e = threadIdx.x; e < tot; e += blockDim.x) {
-        const int x = e / w, r = e - x * w;
-        base[x * xstride + r] = sl[e];
-    }
-}
-
 // ---------------------------------------------- x pass of the check FFT
 // eqVar partials: mechanical sums kz >= 1 of sqrt|sum_c |s_c|^2 W_c| with
 // W = (xi0^2, xi1^2, xi2^2, 2xi1+2xi2, 2xi0+2xi2, 2xi0+2xi1) (FFT_analysis3D.cpp:366-389);
 // thermal sums kz >= 0 of sqrt(sum_c |q_c|^2 xi_c^2) (FFT_thermal3D.cpp:315-335).
-template <typename T, typename PH, int WHICH, bool GEN>
-__global__ void __launch_bounds__(XYTHREADS) k_xcheck(Geo g, Ptr<T> p)
+// The term of frequency (kx, y, kz) with values v; a2: |v_c|^2.
+template <typename T, int C>
+__device__ __forceinline__ double eq_term(const Geo& g, int kx, int y, int kz, const cx<T>* v, double (&a2)[C])
 {
-    extern __shared__ __align__(16) unsigned char smem_raw[];
-    __shared__ double red[XYTHREADS / 64];
-    cx<T>* sl = reinterpret_cast<cx<T>*>(smem_raw);
-    constexpr int C = PH::C;
-    const int per = g.Ny * g.nkx;
-    const int s = blockIdx.x / per;
-    const int t = blockIdx.x % per;
-    const int y = t / g.nkx;
-    const int kz0 = (t % g.nkx) * g.TKx;
-    const Ctl& ctl = p.ctl[s];
-    if (ctl.done) return;
-    if (WHICH == BUF_CHK_CUR && !ctl.need_cur) return;
-    if (WHICH == BUF_CHK_PREV && !ctl.need_prev) return;
-    const int nk = min(g.TKx, g.Nzh - kz0);
-    const int w = nk * C;
-    const cx<T>* base = p.K + (long long)s * p.sS + ((long long)y * g.Nzh + kz0) * C;
-    const long long xstride = (long long)g.Ny * g.Nzh * C;
-    const int tot = g.Nx * w;
-    for (int e = threadIdx.x; e < tot; e += blockDim.x) {
-        const int x = e / w, r = e - x * w;
-        sl[e] = base[x * xstride + r];
-    }
-    __syncthreads();
-    fft_lines<T, -1, EPT, true, GEN>(sl, LineGeo{w, w, 1, 0, w}, g.ax, p.twx);
-    double acc = 0.0;
-    for (int f = threadIdx.x; f < g.Nx * nk; f += blockDim.x) {
-        const int kx = f / nk, kzl = f - kx * nk;
-        const int kz = kz0 + kzl;
-        const cx<T>* v = sl + kx * w + kzl * C;
-        double a2[C];
 #pragma unroll
-        for (int c = 0; c < C; ++c) a2[c] = (double)v[c].re * (double)v[c].re + (double)v[c].im * (double)v[c].im;
-        if constexpr (C == 6) {
-            if (kz >= 1) {
-                const double z0 = Elastic::fmap(kz, g.Nz), z1 = Elastic::fmap(y, g.Ny), z2 = Elastic::fmap(kx, g.Nx);
-                const double q = a2[0] * z0 * z0 + a2[1] * z1 * z1 + a2[2] * z2 * z2 + a2[3] * ((z1 + z1) + (z2 + z2)) +
-                                 a2[4] * ((z0 + z0) + (z2 + z2)) + a2[5] * ((z0 + z0) + (z1 + z1));
-                acc += sqrt(fabs(q));
-            }
-        } else {
-            const double z0 = fmap_t(kz, g.Nz), z1 = fmap_t(y, g.Ny), z2 = fmap_t(kx, g.Nx);
-            acc += sqrt(a2[0] * z0 * z0 + a2[1] * z1 * z1 + a2[2] * z2 * z2);
-        }
-        if (kx == 0 && y == 0 && kz == 0) {
-            double dd;
-            if constexpr (C == 6) dd = sqrt(a2[0] + a2[1] + a2[2] + 2 * a2[3] + 2 * a2[4] + 2 * a2[5]);
-            else dd = sqrt(a2[0] + a2[1] + a2[2]);
-            p.pchk[((long long)s * 2 + (WHICH == BUF_CHK_CUR ? 0 : 1)) * (g.nbc + 1) + g.nbc] = dd;
-        }
+    for (int c = 0; c < C; ++c) a2[c] = (double)v[c].re * (double)v[c].re + (double)v[c].im * (double)v[c].im;
+    if constexpr (C == 6) {
+        if (kz < 1) return 0.0;
+        const double z0 = Elastic::fmap(kz, g.Nz), z1 = Elastic::fmap(y, g.Ny), z2 = Elastic::fmap(kx, g.Nx);
+        const double q = a2[0] * z0 * z0 + a2[1] * z1 * z1 + a2[2] * z2 * z2 + a2[3] * ((z1 + z1) + (z2 + z2)) +
+                         a2[4] * ((z0 + z0) + (z2 + z2)) + a2[5] * ((z0 + z0) + (z1 + z1));
+        return sqrt(fabs(q));
+    } else {
+        const double z0 = fmap_t(kz, g.Nz), z1 = fmap_t(y, g.Ny), z2 = fmap_t(kx, g.Nx);
+        return sqrt(a2[0] * z0 * z0 + a2[1] * z1 * z1 + a2[2] * z2 * z2);
     }
-    const double bs = block_sum(acc, red);
-    if (threadIdx.x == 0) p.pchk[((long long)s * 2 + (WHICH == BUF_CHK_CUR ? 0 : 1)) * (g.nbc + 1) + t] = bs;
+}
+
+// the norm of the mean field from its |v_c|^2 at the zero frequency
+template <int C>
+__device__ __forceinline__ double eq_mean(const double (&a2)[C])
+{
+    if constexpr (C == 6) return sqrt(a2[0] + a2[1] + a2[2] + 2 * a2[3] + 2 * a2[4] + 2 * a2[5]);
+    else return sqrt(a2[0] + a2[1] + a2[2]);
 }
 
 // ---------------------------------------------------------- finalizers
@@ -921,29 +580,6 @@ __global__ void k_promote(Geo g, Ptr<float> p32, Ptr<double> p64, const Ctl* ctl
         double* dst = u_buf(p64, it, s);
         for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x)
             dst[i] = (double)src[i];
-    }
-}
-
-// start of the anchored polish, after one FP64 iteration from the anchor
-// A = iterate it-1: r = T(A) - A = u[it] - u[it-1] (FP64 difference, kept
-// in FP32), and the correction of iterate `it` is e = r.  Skips solves that
-// are done or not anchored.
-template <int C>
-__global__ void k_anchor(Geo g, Ptr<double> p64, Ptr<float> p32, const Ctl* ctl)
-{
-    const long long n = g.N * C;
-    for (int s = 0; s < g.nsolve; ++s) {
-        if (ctl[s].done || !ctl[s].corr) continue;
-        const int it = ctl[s].it;
-        const double* a = u_buf(p64, it - 1, s);
-        const double* b = u_buf(p64, it, s);
-        float* e = u_buf(p32, it, s);
-        float* r = const_cast<float*>(p32.R) + (long long)s * p32.sU;
-        for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x) {
-            const float d = (float)(b[i] - a[i]);
-            e[i] = d;
-            r[i] = d;
-        }
     }
 }
 
