@@ -253,16 +253,20 @@ __global__ void __launch_bounds__(FTHREADS) k_bfin1(Geo g, Ctl* ctl, const doubl
     }
 }
 
-// after the x pass: eqVar of this iterate, diff_avr_eqVar, stop rule (:820-826)
+// after the x pass: eqVar of this iterate, diff_avr_eqVar, stop rule (:820-826);
+// hs: the iterations' published state (publish)
 template <int U = 0> // a template so that every unit including this header may instantiate it
-__global__ void __launch_bounds__(FTHREADS) k_bfin2(Geo g, Ctl* ctl, const double* pchk)
+__global__ void __launch_bounds__(FTHREADS) k_bfin2(Geo g, Ctl* ctl, const double* pchk, unsigned long long* hs)
 {
     __shared__ double red[FTHREADS / 64];
     const int s = blockIdx.x;
     Ctl& c = ctl[s];
     const int done = c.done;
     __syncthreads();
-    if (done) return;
+    if (done) {
+        if (threadIdx.x == 0) publish(c, hs, s);
+        return;
+    }
     const double* pc = pchk + (long long)s * (g.nbx + 1);
     const double cc = ordered_sum(pc, g.nbx, red);
     if (threadIdx.x == 0) {
@@ -281,6 +285,7 @@ __global__ void __launch_bounds__(FTHREADS) k_bfin2(Geo g, Ctl* ctl, const doubl
         if (c.err) c.done = 3;
         else if (c.it > 1 && fabs(c.deq) < c.tol_eq && fabs(c.dsum) < c.tol_f) c.done = 1;
         else if (c.it > c.cap) c.done = 2;
+        publish(c, hs, s);
     }
 }
 

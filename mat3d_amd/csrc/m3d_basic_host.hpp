@@ -43,6 +43,8 @@ struct BasicRunner {
     double* bs = nullptr;
     double* mat = nullptr;
     Ctl* ctl = nullptr;
+    Ctl cfin{};                       // control block of the FINAL pass
+    unsigned long long* hs = nullptr; // pinned: the solve's published state
     int nblk = 256;
     std::vector<double> prop; // rows x 9, column-major like prop_homogenized
     int rows = 0;
@@ -96,6 +98,7 @@ struct BasicRunner {
             e.alloc(&bs, sizeof(double) * 14 * nblk);
             e.alloc(&mat, sizeof(double) * 256 * 8);
             e.alloc(&ctl, sizeof(Ctl));
+            HCHK(hipHostMalloc((void**)&hs, sizeof(*hs), hipHostMallocMapped | hipHostMallocCoherent));
             two = fp32 && fast;
             if (two) {
                 e.alloc(&f6s, sizeof(float) * 24 * N);
@@ -114,6 +117,8 @@ struct BasicRunner {
         for (void* q : {(void*)f6, (void*)f1, (void*)S6, (void*)S12, (void*)Eh, (void*)psum, (void*)psum2, (void*)pfin, (void*)pchk,
                         (void*)bs, (void*)mat, (void*)ctl, (void*)f6s, (void*)f1s, (void*)S6s, (void*)S12s, (void*)Ehs})
             if (q) (void)hipFree(q);
+        if (hs) (void)hipHostFree(hs);
+        hs = nullptr;
         f6 = f1 = psum = psum2 = pfin = pchk = bs = mat = nullptr;
         S6 = S12 = Eh = nullptr;
         f6s = f1s = nullptr;
@@ -226,37 +231,54 @@ struct BasicRunner {
             flex::launch_y<T>(-1, BUF_K, 0, g, yp, st);
             bflex::launch_x(g, bp, st, iter);
         }
-        hipLaunchKernelGGL((k_bfin2<0>), dim3(1), dim3(FTHREADS), 0, st, g, ctl, pchk);
+        hipLaunchKernelGGL((k_bfin2<0>), dim3(1), dim3(FTHREADS), 0, st, g, ctl, pchk, iter ? hs : nullptr);
         if (fast) bfast::launch_y6<T>(gf6, yp, st);
         else if constexpr (sizeof(T) == 8)
             flex::launch_y<T>(1, BUF_MAIN, 0, g6, yp, st);
     }
 
     // the fields and state of the increment's last iterate on the FP64 path,
-    // whose iterations do not store them: the z pass
-    // in FINAL mode on the S6 buffer that iterate was computed from (for
-    // "ep" it also leaves the export sums in pfin and applies
-    // update_old_Variable).  The
-    // iterations after the start stage (itNo it0) alternate the buffers from
-    // buffer 0, so iterate itNo c.it read buffer (c.it - it0 - 1) & 1.  The
-    // z pass skips a solve marked done, so the flag is cleared around it; c
-    // is the host copy of the control block after the iterations.
-    void finish(Ctl& c, int it0)
+    // whose iterations do not store them: the z pass in FINAL mode on the S6
+    // buffer that iterate was computed from (for "ep" it also leaves the export
+    // sums in pfin and applies update_old_Variable).  The iterations after the
+    // start stage (itNo it0) alternate the buffers from buffer 0, so iterate
+    // itNo c.it read buffer (c.it - it0 - 1) & 1.  The z pass skips a solve
+    // marked done, so the flag is cleared for it; c is the host copy of the
+    // control block after the iterations.
+    void finish(const Ctl& c, int it0)
     {
         hipStream_t st = e.st;
-        Ctl run = c;
-        run.done = 0;
-        HCHK(hipMemcpyAsync(ctl, &run, sizeof run, hipMemcpyHostToDevice, st));
+        cfin = c;
+        cfin.done = 0;
+        HCHK(hipMemcpyAsync(ctl, &cfin, sizeof cfin, hipMemcpyHostToDevice, st));
         const BPtr<double> bp = bptr_t<double>((c.it - it0 - 1) & 1);
         if (fast) bfast::launch_z<double>(beh, BMODE_FINAL, gf, bp, st, lin);
         else bflex::launch_z(beh, BMODE_FINAL, g6, bp, st, lin);
         HCHK(hipGetLastError());
-        Ctl after;
-        HCHK(hipMemcpyAsync(&after, ctl, sizeof after, hipMemcpyDeviceToHost, st));
+    }
+
+    // iterations after a start stage until the stop rule holds, one queued
+    // ahead of the state the host has read; c: the device's control block
+    // (whose tick starts at 0)
+    template <typename T>
+    void iterate(Ctl& c)
+    {
+        hipStream_t st = e.st;
+        for (unsigned long long k = 0;; ++k) {
+            stage<T>(BMODE_ITER, (int)(k & 1));
+            HCHK(hipGetLastError());
+            if (k > 0 && wait_ticks(st, hs, 1, k)) break;
+        }
+        HCHK(hipMemcpyAsync(&c, ctl, sizeof c, hipMemcpyDeviceToHost, st));
         HCHK(hipStreamSynchronize(st));
-        if (after.err) c.done = 3;
-        HCHK(hipMemcpyAsync(ctl, &c, sizeof c, hipMemcpyHostToDevice, st));
-        HCHK(hipStreamSynchronize(st));
+    }
+
+    // upload the control block and the state words it starts from
+    void load_ctl(Ctl& c)
+    {
+        c.tick = 0;
+        *hs = 0;
+        HCHK(hipMemcpyAsync(ctl, &c, sizeof c, hipMemcpyHostToDevice, e.st));
     }
 
     // mtab: per phase {la, mu, Sy, H, n, P, Y0, 0}; la0/mu0: reference medium;
@@ -294,47 +316,15 @@ struct BasicRunner {
         rows = nInc;
         exit_inc = -1;
         int nx = 0, total_it = 0, total32 = 0;
+        const ArgError newton{M3D_ERR_NUMERIC, "constitutive update: Newton iteration failed (NaN or no convergence)"};
         std::vector<double> part((size_t)14 * nblk);
-        const int ck = 4;
-        // captured graphs of `ck` iterations (FP64, and FP32 for the FP32
-        // phase), replayed in every increment
-        struct GraphGuard {
-            hipGraph_t g = nullptr;
-            hipGraphExec_t x = nullptr;
-            ~GraphGuard()
-            {
-                if (x) (void)hipGraphExecDestroy(x);
-                if (g) (void)hipGraphDestroy(g);
-            }
-        } g64, g32;
-        auto capture = [&](GraphGuard& gg, bool fp32) {
-            HCHK(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
-            for (int k = 0; k < ck; ++k) {
-                if (fp32) stage<float>(BMODE_ITER, k & 1);
-                else stage(BMODE_ITER, k & 1);
-            }
-            HCHK(hipStreamEndCapture(st, &gg.g));
-            hipError_t ge = hipGraphInstantiate(&gg.x, gg.g, nullptr, nullptr, 0);
-            if (ge != hipSuccess) throw HipError{ge, "hipGraphInstantiate"};
-        };
-        capture(g64, false);
-        if (two) capture(g32, true);
-        auto replay = [&](hipGraphExec_t x) {
-            for (int guard = 0; guard < 100000; ++guard) {
-                HCHK(hipGraphLaunch(x, st));
-                HCHK(hipMemcpyAsync(&c, ctl, sizeof c, hipMemcpyDeviceToHost, st));
-                HCHK(hipStreamSynchronize(st));
-                if (c.done) break;
-            }
-        };
         BPtr<float> bp32{};
         if (two) bp32 = bptr_t<float>();
         const int nb = 1024;
         HCHK(hipEventRecord(e.ev0, st));
         for (int inc = 0; inc < nInc; ++inc) {
-            // host copy of the device state, then reset the per-increment fields
-            HCHK(hipMemcpyAsync(&c, ctl, sizeof c, hipMemcpyDeviceToHost, st));
-            HCHK(hipStreamSynchronize(st));
+            // c: the device's state after the previous increment; reset the
+            // per-increment fields
             c.incNo = inc + 1;
             c.done = 0;
             c.it = 0;
@@ -345,12 +335,12 @@ struct BasicRunner {
                 // FP32 phase from the increment's FP64 start state
                 c.tol_f = std::max(tol_f * e.polish_factor, e.fp32_floor);
                 c.tol_eq = std::max(tol_eq * e.polish_factor, e.fp32_floor);
-                HCHK(hipMemcpyAsync(ctl, &c, sizeof c, hipMemcpyHostToDevice, st));
+                load_ctl(c);
                 hipLaunchKernelGGL((k_bcopy<double, float>), dim3(nb), dim3(256), 0, st, g12, bp, bp32,
                                    BC_EPS | BC_SIGOLD | BC_EPSOLD | BC_EP);
                 stage<float>(BMODE_START, 1);
                 HCHK(hipGetLastError());
-                replay(g32.x);
+                iterate<float>(c);
                 if (c.done == 2) {
                     // iteration cap reached in FP32: that state is the result
                     hipLaunchKernelGGL((k_bcopy<float, double>), dim3(nb), dim3(256), 0, st, g12, bp32, bp,
@@ -368,10 +358,10 @@ struct BasicRunner {
                     c.tol_f = tol_f;
                     c.tol_eq = tol_eq;
                     const int it0 = c.it;
-                    HCHK(hipMemcpyAsync(ctl, &c, sizeof c, hipMemcpyHostToDevice, st));
+                    load_ctl(c);
                     stage<double>(BMODE_RESTART, 1);
                     HCHK(hipGetLastError());
-                    replay(g64.x);
+                    iterate<double>(c);
                     if (c.done != 3) {
                         finish(c, it0);
                         fused = beh == BEH_EP;
@@ -388,17 +378,16 @@ struct BasicRunner {
             if (fp64_run) {
                 c.tol_f = tol_f;
                 c.tol_eq = tol_eq;
-                HCHK(hipMemcpyAsync(ctl, &c, sizeof c, hipMemcpyHostToDevice, st));
+                load_ctl(c);
                 stage(BMODE_START, 1);
                 HCHK(hipGetLastError());
-                replay(g64.x);
+                iterate<double>(c);
                 if (c.done != 3) {
                     finish(c, 0);
                     fused = beh == BEH_EP;
                 }
             }
-            if (c.done == 3)
-                throw ArgError{M3D_ERR_NUMERIC, "constitutive update: Newton iteration failed (NaN or no convergence)"};
+            if (c.done == 3) throw newton;
             total_it += c.it;
             info.iterations = c.it;
             info.status = c.done;
@@ -415,7 +404,10 @@ struct BasicRunner {
                 hipLaunchKernelGGL((k_bsums<double, BEH_ED>), dim3(nblk, 1), dim3(256), 0, st, g12, bp, bs, nblk);
             HCHK(hipGetLastError());
             HCHK(hipMemcpyAsync(part.data(), bs, sizeof(double) * part.size(), hipMemcpyDeviceToHost, st));
+            Ctl after;
+            HCHK(hipMemcpyAsync(&after, ctl, sizeof after, hipMemcpyDeviceToHost, st));
             HCHK(hipStreamSynchronize(st));
+            if (after.err) throw newton; // in the FINAL pass
             double m[14];
             for (int q = 0; q < 14; ++q) {
                 double a = 0;

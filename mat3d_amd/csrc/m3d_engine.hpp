@@ -2,11 +2,10 @@
 // m3d_engine.hpp -- host runtime of libmat3d.so (gfx950), shared by the ABI units.
 //
 // Owns the device state of one solver handle, builds the FFT plans and tile
-// shapes, drives the iteration as captured hipGraphs of a chunk of
-// iterations and assembles the homogenized tensors in FP64 on the host.
-// Control decisions (stop rule, equilibrium-check scheduling) are taken on
-// the device; the host only polls the per-solve done flags between graph
-// replays.
+// shapes, launches the iterations and assembles the homogenized tensors in
+// FP64 on the host.  Control decisions (stop rule, need of an equilibrium
+// check) are taken on the device; the host reads the solves' state one
+// iteration behind and launches with or without the check passes.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -19,6 +18,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include <sys/stat.h>
@@ -180,6 +180,30 @@ Geo make_geo(int Nx, int Ny, int Nz, int C)
     }
     g.spec = (long long)((Nx - 1) >> g.lxb) * g.sxa + (long long)((Nx - 1) & g.xbm) * g.sxb + (long long)(Ny - 1) * g.sy + rowc;
     return g;
+}
+
+// wait until the n solves of hs have published `ticks` states each; true if
+// all of them are done
+inline bool wait_ticks(hipStream_t st, const unsigned long long* hs, int n, unsigned long long ticks)
+{
+    bool all = true;
+    for (int s = 0; s < n; ++s) {
+        unsigned long long v;
+        for (int spin = 1; ((v = __atomic_load_n(hs + s, __ATOMIC_RELAXED)) >> 8) < ticks; ++spin) {
+            if (spin % 256) continue;
+            // an idle or failed stream publishes nothing more
+            const hipError_t q = hipStreamQuery(st);
+            if (q == hipErrorNotReady) {
+                std::this_thread::yield();
+            } else if (q != hipSuccess) {
+                throw HipError{q, "hipStreamQuery"};
+            } else if ((__atomic_load_n(hs + s, __ATOMIC_RELAXED) >> 8) < ticks) {
+                throw ArgError{M3D_ERR_HIP, "the device stopped without publishing its state"};
+            }
+        }
+        all = all && (v & ST_DONE);
+    }
+    return all;
 }
 
 // ---------------------------------------------------------- small algebra
@@ -387,6 +411,7 @@ struct Engine {
     double* fbuf = nullptr; // field output staging (2*C*N doubles)
     hipStream_t st = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
+    unsigned long long* hstate = nullptr; // pinned: the solves' published states (publish)
     // host state
     int nsolve = 0;
     std::vector<int> final_prec; // per solve: 0 fp32, 1 fp64
@@ -401,7 +426,7 @@ struct Engine {
     double rollback_margin = 2.0;
     double fp32_floor = 1e-6;
     int cap = 2000;
-    int chunk = 0;
+    int chunk = 0; // iterations launched between two looks at the state (0: 1)
     int mnblk = 256;
 
     Engine(int nx, int ny, int nz, int prec) : Nx(nx), Ny(ny), Nz(nz), precision(prec)
@@ -440,6 +465,8 @@ struct Engine {
         if (psum) hipFree(psum);
         if (pchk) hipFree(pchk);
         if (ctl) hipFree(ctl);
+        if (hstate) hipHostFree(hstate);
+        hstate = nullptr;
         if (mpart) hipFree(mpart);
         if (rve_of) hipFree(rve_of);
         Sbuf = Kbuf = nullptr;
@@ -516,6 +543,7 @@ struct Engine {
         alloc(&psum, sizeof(double) * (size_t)nbz * n);
         alloc(&pchk, sizeof(double) * (size_t)2 * (nbx + 1) * n);
         alloc(&ctl, sizeof(Ctl) * n);
+        HCHK(hipHostMalloc((void**)&hstate, sizeof(*hstate) * n, hipHostMallocMapped | hipHostMallocCoherent));
         alloc(&mpart, sizeof(double) * (size_t)2 * C * mnblk * n);
         alloc(&rve_of, sizeof(int) * n);
         std::vector<int> z(n, 0);
@@ -749,40 +777,47 @@ struct Engine {
         ypass<T, 1, BUF_MAIN>(g, p);
     }
 
-    // green = false: the iteration's update and stop check only, without the
-    // transforms that prepare the next iteration's Green output (the FP64
-    // anchor iteration of the polish, which the FP32 corrections follow)
+    // the equilibrium-check passes an iteration holds (CHECKS_*) and the stop rule
     template <typename T>
-    void launch_iter(const Geo& g, const Ptr<T>& p, bool green = true)
+    void launch_checks(const Geo& g, const Ptr<T>& p, int checks, unsigned long long* hs)
     {
-        // the FP64 anchor iteration also writes r and e (MODE_IUA)
-        if constexpr (sizeof(T) == 8) {
-            if (!green) zpass<T, MODE_IUA>(g, p);
-            else zpass<T, MODE_IUF>(g, p);
-        } else {
-            zpass<T, MODE_IUF>(g, p);
-        }
-        hipLaunchKernelGGL((k_finA<C>), dim3(g.nsolve), dim3(fin_threads(g.nbz)), 0, st, g, p.ctl, p.psum);
+        if (checks == CHECKS_NONE) return;
         zpass<T, MODE_CHK_CUR>(g, p);
         ypass<T, -1, BUF_CHK_CUR>(g, p);
         xcheck<T, BUF_CHK_CUR>(g, p);
-        zpass<T, MODE_CHK_PREV>(g, p);
-        ypass<T, -1, BUF_CHK_PREV>(g, p);
-        xcheck<T, BUF_CHK_PREV>(g, p);
-        hipLaunchKernelGGL((k_finB<C>), dim3(g.nsolve), dim3(fin_threads(g.nbc)), 0, st, g, p.ctl, p.pchk);
-        if (!green) return;
+        if (checks == CHECKS_BOTH) {
+            zpass<T, MODE_CHK_PREV>(g, p);
+            ypass<T, -1, BUF_CHK_PREV>(g, p);
+            xcheck<T, BUF_CHK_PREV>(g, p);
+        }
+        hipLaunchKernelGGL((k_finB<C>), dim3(g.nsolve), dim3(fin_threads(g.nbc)), 0, st, g, p.ctl, p.pchk, hs);
+    }
+
+    template <typename T>
+    void launch_finA(const Geo& g, const Ptr<T>& p, int checks, unsigned long long* hs)
+    {
+        hipLaunchKernelGGL((k_finA<C>), dim3(g.nsolve), dim3(fin_threads(g.nbz)), 0, st, g, p.ctl, p.psum, checks, hs);
+    }
+
+    template <typename T>
+    void launch_iter(const Geo& g, const Ptr<T>& p, int checks)
+    {
+        zpass<T, MODE_IUF>(g, p);
+        launch_finA(g, p, checks, hstate);
+        launch_checks(g, p, checks, hstate);
         ypass<T, -1, BUF_MAIN>(g, p);
         xgreen<T>(g, p);
         ypass<T, 1, BUF_MAIN>(g, p);
     }
 
-    int chunk_for(const Geo& g) const
+    // the FP64 anchor iteration of the polish: update (which also writes r and
+    // e, MODE_IUA) and stop check, without the transforms that would prepare
+    // its successor's Green output (the FP32 corrections follow)
+    void launch_anchor(const Geo& g, const Ptr<double>& p)
     {
-        if (chunk > 0) return chunk;
-        const double work = (double)g.N * g.nsolve;
-        if (work >= 3.0e7) return 2;
-        if (work >= 4.0e6) return 4;
-        return 8;
+        zpass<double, MODE_IUA>(g, p);
+        launch_finA(g, p, CHECKS_BOTH, nullptr);
+        launch_checks(g, p, CHECKS_BOTH, nullptr);
     }
 
     // anchored polish: FP32 passes on the corrections e (r added in the
@@ -796,54 +831,53 @@ struct Engine {
         ypass<float, 1, BUF_MAIN>(gf, pf);
     }
 
-    void launch_iter_corr(const Geo& gf, const Ptr<float>& pf, const Geo& gd, const Ptr<double>& pd)
+    void launch_iter_corr(const Geo& gf, const Ptr<float>& pf, const Geo& gd, const Ptr<double>& pd, int checks)
     {
         zpass<float, MODE_IUFR>(gf, pf);
-        hipLaunchKernelGGL((k_finA<C>), dim3(gf.nsolve), dim3(fin_threads(gf.nbz)), 0, st, gf, pf.ctl, pf.psum);
-        zpass<double, MODE_CHK_CUR>(gd, pd);
-        ypass<double, -1, BUF_CHK_CUR>(gd, pd);
-        xcheck<double, BUF_CHK_CUR>(gd, pd);
-        zpass<double, MODE_CHK_PREV>(gd, pd);
-        ypass<double, -1, BUF_CHK_PREV>(gd, pd);
-        xcheck<double, BUF_CHK_PREV>(gd, pd);
-        hipLaunchKernelGGL((k_finB<C>), dim3(gd.nsolve), dim3(fin_threads(gd.nbc)), 0, st, gd, pd.ctl, pd.pchk);
+        launch_finA(gf, pf, checks, hstate);
+        launch_checks(gd, pd, checks, hstate);
         ypass<float, -1, BUF_MAIN>(gf, pf);
         xgreen<float>(gf, pf);
         ypass<float, 1, BUF_MAIN>(gf, pf);
     }
 
-    // capture `ck` iterations (iter()) in a graph and replay it until every
-    // solve of the batch is done; the host polls the done flags in between
-    template <typename Iter>
-    void run_graph(int ck, Iter&& iter, std::vector<Ctl>& hctl)
+    // The checks the next launched iterations have to hold, from the newest
+    // published state of the solves: none while no running solve is near its
+    // stop, the current iterate's alone where every solve that is has a checked
+    // iterate behind it.  A guess only: a solve that needs more than it was
+    // given waits (k_finA).
+    int checks_for() const
     {
-        hipGraph_t graph = nullptr;
-        hipGraphExec_t exec = nullptr;
-        HCHK(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
-        for (int i = 0; i < ck; ++i) iter();
-        hipError_t ce = hipStreamEndCapture(st, &graph);
-        if (ce != hipSuccess) throw HipError{ce, "hipStreamEndCapture"};
-        ce = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
-        if (ce != hipSuccess) {
-            hipGraphDestroy(graph);
-            throw HipError{ce, "hipGraphInstantiate"};
+        int need = CHECKS_NONE;
+        for (int s = 0; s < nsolve; ++s) {
+            const unsigned long long v = __atomic_load_n(hstate + s, __ATOMIC_RELAXED);
+            if ((v & ST_DONE) || !(v & (ST_WAIT | ST_NEAR))) continue;
+            if ((v & ST_WAIT) || !(v & ST_CHECKED)) return CHECKS_BOTH;
+            need = CHECKS_CUR;
         }
-        try {
-            for (int guard = 0; guard < 100000; ++guard) {
-                HCHK(hipGraphLaunch(exec, st));
-                HCHK(hipMemcpyAsync(hctl.data(), ctl, sizeof(Ctl) * nsolve, hipMemcpyDeviceToHost, st));
-                HCHK(hipStreamSynchronize(st));
-                bool all = true;
-                for (int s = 0; s < nsolve; ++s) all = all && hctl[s].done;
-                if (all) break;
-            }
-        } catch (...) {
-            hipGraphExecDestroy(exec);
-            hipGraphDestroy(graph);
-            throw;
+        return need;
+    }
+
+    // Launch iterations (iter(checks), ck at a time) until every solve of the
+    // batch is done.  The host stays one group of launches ahead: it reads the
+    // state after one while the next runs, so the device does not wait for it
+    // (what was queued when the last solve ended only skips).  Plain launches:
+    // they cost the host 3-4.5 us each and a kernel of the smallest grids takes
+    // 4-12 us, while capturing and instantiating a graph took 50 us (12 nodes)
+    // to 800 us (80 nodes) in every call, and the device 8 us between graphs.
+    // The control blocks' ticks start at 0.
+    template <typename Iter>
+    void run_loop(int ck, Iter&& iter, std::vector<Ctl>& hctl)
+    {
+        std::fill(hstate, hstate + nsolve, 0ull);
+        for (unsigned long long k = 0;; ++k) {
+            const int checks = checks_for();
+            for (int i = 0; i < ck; ++i) iter(checks);
+            HCHK(hipGetLastError());
+            if (k > 0 && wait_ticks(st, hstate, nsolve, k * ck)) break;
         }
-        hipGraphExecDestroy(exec);
-        hipGraphDestroy(graph);
+        HCHK(hipMemcpyAsync(hctl.data(), ctl, sizeof(Ctl) * nsolve, hipMemcpyDeviceToHost, st));
+        HCHK(hipStreamSynchronize(st));
     }
 
     // run the iteration in precision T until every solve of the batch is done
@@ -854,7 +888,7 @@ struct Engine {
         Ptr<T> p = ptrs<T>(g);
         launch_start<T>(g, p);
         HCHK(hipGetLastError());
-        run_graph(chunk_for(g), [&]() { launch_iter<T>(g, p); }, hctl);
+        run_loop(std::max(1, chunk), [&](int checks) { launch_iter<T>(g, p, checks); }, hctl);
     }
 
     // anchored polish of the solves flagged corr (r and e from the anchor
@@ -866,7 +900,7 @@ struct Engine {
         Ptr<double> pd = ptrs<double>(gd);
         launch_start_corr(gf, pf);
         HCHK(hipGetLastError());
-        run_graph(chunk_for(gf), [&]() { launch_iter_corr(gf, pf, gd, pd); }, hctl);
+        run_loop(std::max(1, chunk), [&](int checks) { launch_iter_corr(gf, pf, gd, pd, checks); }, hctl);
     }
 
     // time the FP32 x/y pass variants on this shape (first FP32 solve); the
@@ -1051,7 +1085,7 @@ struct Engine {
                 }
                 hctl[s].it = jr[s];
                 hctl[s].done = 0;
-                hctl[s].need_cur = hctl[s].need_prev = 0;
+                hctl[s].need_cur = hctl[s].need_prev = hctl[s].wait = hctl[s].tick = 0;
                 hctl[s].eq_it = -1;
                 hctl[s].tol_f = tol_f;
                 hctl[s].tol_eq = tol_eq;
@@ -1071,7 +1105,7 @@ struct Engine {
                 // so that iteration stops after its update and stop check.
                 Ptr<double> pd = ptrs<double>(gd);
                 launch_start<double>(gd, pd, true);
-                launch_iter<double>(gd, pd, false);
+                launch_anchor(gd, pd);
                 HCHK(hipGetLastError());
                 HCHK(hipMemcpyAsync(hctl.data(), ctl, sizeof(Ctl) * nsolve, hipMemcpyDeviceToHost, st));
                 HCHK(hipStreamSynchronize(st));
@@ -1182,6 +1216,7 @@ struct Engine {
             c.done = 0;
             c.need_cur = 1;
             c.need_prev = 1;
+            c.wait = 0;
             c.corr = 0;
         }
         HCHK(hipMemcpy(ctl, hctl.data(), sizeof(Ctl) * nsolve, hipMemcpyHostToDevice));

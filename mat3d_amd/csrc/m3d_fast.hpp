@@ -628,7 +628,7 @@ __device__ __forceinline__ void kz_tile(const Geo& g, const Ptr<T>& p, int b, cx
     constexpr bool ANC = MODE == MODE_IUA; // anchor iteration: no forward transform
     constexpr bool CHK = MODE == MODE_CHK_CUR || MODE == MODE_CHK_PREV;
     const Ctl& ctl = p.ctl[s];
-    if (ctl.done) return;
+    if (ctl.done || ctl.wait) return;
     if (MODE == MODE_CHK_CUR && !ctl.need_cur) return;
     if (MODE == MODE_CHK_PREV && !ctl.need_prev) return;
     const int it = ctl.it;
@@ -847,7 +847,7 @@ __device__ __forceinline__ void kz_tile(const Geo& g, const Ptr<T>& p, int b, cx
 template <int WHICH>
 __device__ __forceinline__ bool chk_needed(const Ctl& c)
 {
-    return !c.done && (WHICH == BUF_CHK_CUR ? c.need_cur : c.need_prev);
+    return !c.done && !c.wait && (WHICH == BUF_CHK_CUR ? c.need_cur : c.need_prev);
 }
 
 // The main passes run one workgroup per tile.  The check passes run a capped
@@ -986,7 +986,7 @@ __device__ __forceinline__ void xy_tile(const Geo& g, const Ptr<T>& p, const Ctl
 template <int WHICH>
 __device__ __forceinline__ bool xy_active(const Ctl& c)
 {
-    if (c.done) return false;
+    if (c.done || c.wait) return false;
     if (WHICH == BUF_CHK_CUR && !c.need_cur) return false;
     if (WHICH == BUF_CHK_PREV && !c.need_prev) return false;
     return true;

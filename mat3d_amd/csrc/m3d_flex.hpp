@@ -241,7 +241,7 @@ __device__ __forceinline__ void store_tile(const cx<T>* sl, cx<T>* base, long lo
 // ------------------------------------------------------------ y and x passes
 __device__ __forceinline__ bool active(const Ctl& c, int which)
 {
-    return !c.done && (which != BUF_CHK_CUR || c.need_cur) && (which != BUF_CHK_PREV || c.need_prev);
+    return !c.done && !c.wait && (which != BUF_CHK_CUR || c.need_cur) && (which != BUF_CHK_PREV || c.need_prev);
 }
 
 // any solve takes part in a check pass (called by the whole workgroup)
@@ -297,7 +297,7 @@ __global__ void __launch_bounds__(NT) k_xg(Geo g, Ptr<T> p, const T* __restrict_
     const int b = fast::xcd_split(blockIdx.x, gridDim.x, per);
     const int s = b / per, t = b - s * per;
     const Ctl& ctl = p.ctl[s];
-    if (ctl.done) return;
+    if (ctl.done || ctl.wait) return;
     const int y = t / g.nkx, kz0 = (t - y * g.nkx) * g.TKx;
     const int nk = min(g.TKx, g.Nzh - kz0), w = nk * C;
     cx<T>* base = p.S + (long long)s * p.sS + (long long)y * g.sy + (long long)kz0 * C;
@@ -490,7 +490,7 @@ __device__ __forceinline__ void z_tile(const Geo& g, const Ptr<T>& p, int which,
     constexpr bool FWD = MODE == MODE_FWD || MODE == MODE_FWDP;
     const int s = b / g.nbz, t = b - s * g.nbz;
     const Ctl& ctl = p.ctl[s];
-    if (ctl.done || (CHK && !active(ctl, which))) return;
+    if (ctl.done || ctl.wait || (CHK && !active(ctl, which))) return;
     const int it = ctl.it;
     const int x = t / g.nty, y0 = (t - x * g.nty) * g.TY;
     const int ny = min(g.TY, g.Ny - y0);

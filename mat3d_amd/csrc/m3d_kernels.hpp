@@ -58,7 +58,10 @@ struct Ctl {
     // FP32 passes iterate e <- r + M e (r = T(A) - A, load term dropped)
     int corr;
     int anc_it;
-    int pad;
+    // 1: the iterate needs a check that the launched sequence does not hold;
+    // the solve stands still until one that does (k_finA)
+    int wait;
+    int tick; // states published to the host since the loop began (publish)
     double sum_anchor; // sum of the dual field of the anchor (FP64)
     double sum_prev;  // sum of the dual field at iterate `it`
     double eq_val;    // eqVar at iterate eq_it
@@ -498,20 +501,57 @@ __global__ void __launch_bounds__(ATHREADS) k_fin0(Geo g, Ctl* ctl, const double
         c.eq_it = -1;
         c.need_cur = 0;
         c.need_prev = 0;
+        c.wait = 0;
     }
 }
 
+// check passes that follow the update pass in a launched iteration: none, the
+// current iterate's, or also the previous iterate's (which only the first
+// checked iterate of a solve needs)
+enum { CHECKS_NONE = 0, CHECKS_CUR = 1, CHECKS_BOTH = 2 };
+
+// What the host's loop knows of a solve: one word per solve in pinned host
+// memory, (tick << 8) | flags, stored by the last finaliser of an iteration.
+// One relaxed 64-bit store needs no fence, and reading it costs the stream
+// nothing; a copy of the control blocks left the device idle for 18 us each
+// time (9 us before the copy, 4 us of it, 5 us after).
+enum { ST_DONE = 1, ST_WAIT = 2, ST_NEAR = 4, ST_CHECKED = 8 };
+constexpr double NEAR_TOL = 3.0; // "near its stop": Delta-sum below this many tolerances
+
+__device__ __forceinline__ void publish(Ctl& c, unsigned long long* hs, int s)
+{
+    if (!hs) return;
+    c.tick += 1;
+    unsigned long long v = (unsigned long long)c.tick << 8;
+    if (c.done) v |= ST_DONE;
+    if (c.wait) v |= ST_WAIT;
+    if (c.it >= 1 && c.dsum < NEAR_TOL * c.tol_f) v |= ST_NEAR;
+    if (c.eq_it == c.it) v |= ST_CHECKED;
+    __hip_atomic_store(hs + s, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // after the update pass: itNo += 1, diff_sum_field, decide whether the
-// equilibrium check is needed (FFT_analysis3D.cpp:392-416, stop rule :785-792)
+// equilibrium check is needed (FFT_analysis3D.cpp:392-416, stop rule :785-792).
+// checks: what this iteration's launches hold.  A solve that needs more waits:
+// every pass of it is skipped until an iteration that holds its checks, which
+// then goes on from the same iterate (its update pass and this decision are
+// not repeated).
 template <int C>
-__global__ void __launch_bounds__(ATHREADS) k_finA(Geo g, Ctl* ctl, const double* psum)
+__global__ void __launch_bounds__(ATHREADS) k_finA(Geo g, Ctl* ctl, const double* psum, int checks, unsigned long long* hs)
 {
     __shared__ double red[ATHREADS / 64];
     const int s = blockIdx.x;
     Ctl& c = ctl[s];
-    const int done = c.done;
+    const int done = c.done, wait = c.wait;
+    if (checks != CHECKS_NONE) hs = nullptr; // k_finB publishes
     __syncthreads();
-    if (done) return;
+    if (done || wait) {
+        if (threadIdx.x == 0) {
+            if (wait && checks >= (c.need_prev ? CHECKS_BOTH : CHECKS_CUR)) c.wait = 0;
+            publish(c, hs, s);
+        }
+        return;
+    }
     const double S0 = ordered_sum(psum + (long long)s * g.nbz, g.nbz, red);
     if (threadIdx.x == 0) {
         const double S = c.corr ? S0 + c.sum_anchor : S0;
@@ -522,20 +562,25 @@ __global__ void __launch_bounds__(ATHREADS) k_finA(Geo g, Ctl* ctl, const double
         const int need = (c.it > 1) && (fabs(c.dsum) < c.tol_f);
         c.need_cur = need;
         c.need_prev = need && (c.eq_it != c.it - 1);
+        c.wait = need && checks < (c.need_prev ? CHECKS_BOTH : CHECKS_CUR);
         if (!need && c.it > c.cap) c.done = 2;
+        publish(c, hs, s);
     }
 }
 
 // after the check FFTs: eqVar, diff_avr_eqVar and the stop decision
 template <int C>
-__global__ void __launch_bounds__(ATHREADS) k_finB(Geo g, Ctl* ctl, const double* pchk)
+__global__ void __launch_bounds__(ATHREADS) k_finB(Geo g, Ctl* ctl, const double* pchk, unsigned long long* hs)
 {
     __shared__ double red[ATHREADS / 64];
     const int s = blockIdx.x;
     Ctl& c = ctl[s];
-    const int done = c.done, need_cur = c.need_cur, need_prev = c.need_prev;
+    const int done = c.done, need_cur = c.need_cur && !c.wait, need_prev = c.need_prev;
     __syncthreads();
-    if (done || !need_cur) return;
+    if (done || !need_cur) {
+        if (threadIdx.x == 0) publish(c, hs, s);
+        return;
+    }
     const double* pc = pchk + (long long)s * 2 * (g.nbc + 1);
     const double cc = ordered_sum(pc, g.nbc, red);
     double ccp = 0;
@@ -551,6 +596,7 @@ __global__ void __launch_bounds__(ATHREADS) k_finB(Geo g, Ctl* ctl, const double
         else if (c.it > c.cap) c.done = 2;
         c.need_cur = 0;
         c.need_prev = 0;
+        publish(c, hs, s);
     }
 }
 
