@@ -405,6 +405,21 @@ __global__ void __launch_bounds__(XNT) M3D_BX_ATTR kxb(Geo g, BPtr<T> p)
     }
 }
 
+// ------------------------------------------------------------------ y pass
+// fast::kxy's y pass; the first workgroup is the finaliser f instead of a tile
+template <typename T, typename PH, int DIR, int WHICH, int L, int TK>
+__global__ void __launch_bounds__(256) kyb(Geo g, Ptr<T> p, BFin f)
+{
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    __shared__ double red[256 / 64][NBSUM];
+    if (blockIdx.x == 0) {
+        bfin_block(p.ctl[0], f, red);
+        return;
+    }
+    fast::xy_body<T, PH, 0, DIR, WHICH, L, TK, 256>(g, p, (const T*)nullptr, fast::xcd_split(blockIdx.x - 1, gridDim.x - 1, gridDim.x - 1),
+                                                    reinterpret_cast<cx<T>*>(smem_raw), &red[0][0]);
+}
+
 // ---------------------------------------------------------------- launchers
 namespace {
 
@@ -431,24 +446,23 @@ void z_mode(const Geo& g, const BPtr<T>& p, hipStream_t st)
 }
 
 template <typename T, typename PH, int DIR, int WHICH, int L>
-bool y_at(const Geo& g, const Ptr<T>& p, hipStream_t st)
+bool y_at(const Geo& g, const Ptr<T>& p, const BFin& f, hipStream_t st)
 {
     if (g.Ny != L) return false;
     constexpr int TK = fast::xytile<T>(L, PH::C);
     const int nkt = (g.Nzh + TK - 1) / TK;
     const size_t sm = ((size_t)L * TK * PH::C + L) * sizeof(cx<T>);
-    hipLaunchKernelGGL((fast::kxy<T, PH, 0, DIR, WHICH, L, TK, 256>), dim3(g.Nx * nkt), dim3(256), sm, st, g, p,
-                       (const T*)nullptr);
+    hipLaunchKernelGGL((kyb<T, PH, DIR, WHICH, L, TK>), dim3(g.Nx * nkt + 1), dim3(256), sm, st, g, p, f);
     return true;
 }
 
 template <typename T, typename PH, int DIR, int WHICH>
-void y_run(const Geo& g, const Ptr<T>& p, hipStream_t st)
+void y_run(const Geo& g, const Ptr<T>& p, const BFin& f, hipStream_t st)
 {
-    const bool ok = y_at<T, PH, DIR, WHICH, 256>(g, p, st) || y_at<T, PH, DIR, WHICH, 192>(g, p, st) ||
-                    y_at<T, PH, DIR, WHICH, 128>(g, p, st) || y_at<T, PH, DIR, WHICH, 96>(g, p, st) ||
-                    y_at<T, PH, DIR, WHICH, 64>(g, p, st) || y_at<T, PH, DIR, WHICH, 48>(g, p, st) ||
-                    y_at<T, PH, DIR, WHICH, 32>(g, p, st);
+    const bool ok = y_at<T, PH, DIR, WHICH, 256>(g, p, f, st) || y_at<T, PH, DIR, WHICH, 192>(g, p, f, st) ||
+                    y_at<T, PH, DIR, WHICH, 128>(g, p, f, st) || y_at<T, PH, DIR, WHICH, 96>(g, p, f, st) ||
+                    y_at<T, PH, DIR, WHICH, 64>(g, p, f, st) || y_at<T, PH, DIR, WHICH, 48>(g, p, f, st) ||
+                    y_at<T, PH, DIR, WHICH, 32>(g, p, f, st);
     if (!ok) throw std::runtime_error("no basic y kernel for this grid");
 }
 
@@ -497,21 +511,21 @@ void launch_z(int beh, int mode, const Geo& g, const BPtr<T>& p, hipStream_t st,
 }
 
 template <typename T>
-void launch_y12(const Geo& g, const Ptr<T>& p, hipStream_t st)
+void launch_y12(const Geo& g, const Ptr<T>& p, const BFin& f, hipStream_t st)
 {
-    y_run<T, Comp12, -1, BUF_K>(g, p, st);
+    y_run<T, Comp12, -1, BUF_K>(g, p, f, st);
 }
 
 template <typename T>
-void launch_y6_fwd(const Geo& g, const Ptr<T>& p, hipStream_t st)
+void launch_y6_fwd(const Geo& g, const Ptr<T>& p, const BFin& f, hipStream_t st)
 {
-    y_run<T, Comp6, -1, BUF_K>(g, p, st);
+    y_run<T, Comp6, -1, BUF_K>(g, p, f, st);
 }
 
 template <typename T>
-void launch_y6(const Geo& g, const Ptr<T>& p, hipStream_t st)
+void launch_y6(const Geo& g, const Ptr<T>& p, const BFin& f, hipStream_t st)
 {
-    y_run<T, Comp6, 1, BUF_MAIN>(g, p, st);
+    y_run<T, Comp6, 1, BUF_MAIN>(g, p, f, st);
 }
 
 template <typename T>
@@ -523,12 +537,12 @@ void launch_x(const Geo& g, const BPtr<T>& p, hipStream_t st, bool e6)
 
 template void launch_z<double>(int, int, const Geo&, const BPtr<double>&, hipStream_t, bool);
 template void launch_z<float>(int, int, const Geo&, const BPtr<float>&, hipStream_t, bool);
-template void launch_y12<double>(const Geo&, const Ptr<double>&, hipStream_t);
-template void launch_y12<float>(const Geo&, const Ptr<float>&, hipStream_t);
-template void launch_y6_fwd<double>(const Geo&, const Ptr<double>&, hipStream_t);
-template void launch_y6_fwd<float>(const Geo&, const Ptr<float>&, hipStream_t);
-template void launch_y6<double>(const Geo&, const Ptr<double>&, hipStream_t);
-template void launch_y6<float>(const Geo&, const Ptr<float>&, hipStream_t);
+template void launch_y12<double>(const Geo&, const Ptr<double>&, const BFin&, hipStream_t);
+template void launch_y12<float>(const Geo&, const Ptr<float>&, const BFin&, hipStream_t);
+template void launch_y6_fwd<double>(const Geo&, const Ptr<double>&, const BFin&, hipStream_t);
+template void launch_y6_fwd<float>(const Geo&, const Ptr<float>&, const BFin&, hipStream_t);
+template void launch_y6<double>(const Geo&, const Ptr<double>&, const BFin&, hipStream_t);
+template void launch_y6<float>(const Geo&, const Ptr<float>&, const BFin&, hipStream_t);
 template void launch_x<double>(const Geo&, const BPtr<double>&, hipStream_t, bool);
 template void launch_x<float>(const Geo&, const BPtr<float>&, hipStream_t, bool);
 

@@ -74,32 +74,34 @@ inline bool supported(int Nx, int Ny, int Nz)
 
 // host launchers (m3d_basic.hip); g carries Nx..Nzh, N, H, invN, nbz, nbx
 // of the tiles above, TY, TKx; the y launch takes the 12- or 6-component
-// view of the spectra in p (S: 6-component Green output, K: 12-component)
+// view of the spectra in p (S: 6-component Green output, K: 12-component) and
+// the finaliser to run beside them
 // (T = double or float)
 // lin: every phase has hardening exponent n = 1 (FP64 "ep" then runs the
 // return map without pow, bit for bit the same arithmetic)
 template <typename T>
 void launch_z(int beh, int mode, const Geo& g, const BPtr<T>& p, hipStream_t st, bool lin = false);
 template <typename T>
-void launch_y12(const Geo& g, const Ptr<T>& p, hipStream_t st);
+void launch_y12(const Geo& g, const Ptr<T>& p, const BFin& f, hipStream_t st);
 // forward y pass of the 6-component sigma^ spectrum that an ITER z pass
 // leaves in the K view
 template <typename T>
-void launch_y6_fwd(const Geo& g, const Ptr<T>& p, hipStream_t st);
+void launch_y6_fwd(const Geo& g, const Ptr<T>& p, const BFin& f, hipStream_t st);
 // e6: the x pass after an ITER z pass (sigma^ with 6 components, eps^ from Eh)
 template <typename T>
 void launch_x(const Geo& g, const BPtr<T>& p, hipStream_t st, bool e6);
 template <typename T>
-void launch_y6(const Geo& g, const Ptr<T>& p, hipStream_t st);
+void launch_y6(const Geo& g, const Ptr<T>& p, const BFin& f, hipStream_t st);
 
 } // namespace bfast
 
 // The same passes for every other grid, in FP64 (m3d_flex_basic.hip): g is a
 // run-time plan of 12 (start stage) or 6 components (iterations, FINAL) whose
-// z and x tiles plan() has set; the y passes are flex::launch_y.
+// z and x tiles plan() has set.
 namespace bflex {
 void plan(Geo& g);
 void launch_z(int beh, int mode, const Geo& g, const BPtr<double>& p, hipStream_t st, bool lin);
+void launch_y(int dir, int which, const Geo& g, const Ptr<double>& p, const BFin& f, hipStream_t st);
 void launch_x(const Geo& g, const BPtr<double>& p, hipStream_t st, bool e6);
 } // namespace bflex
 } // namespace m3d

@@ -36,7 +36,6 @@ struct BasicRunner {
     unsigned char* Ehs = nullptr;
     size_t neh = 0;         // complex values of Eh
     double* psum = nullptr;
-    double* psum2 = nullptr; // [NBSUM][BSPLIT] shares of psum
     double* pfin = nullptr;  // [14][nbz] block sums of the fused FINAL pass
     bool lin = false;        // every phase has hardening exponent n = 1
     double* pchk = nullptr;
@@ -92,7 +91,6 @@ struct BasicRunner {
             neh = fast ? (size_t)gf.nbx * e.Nx * gf.TKx * 6 : (size_t)6 * H;
             e.alloc(&Eh, sizeof(cx<double>) * neh);
             e.alloc(&psum, sizeof(double) * NBSUM * nbz);
-            e.alloc(&psum2, sizeof(double) * NBSUM * BSPLIT);
             e.alloc(&pfin, sizeof(double) * 14 * (size_t)gi().nbz);
             e.alloc(&pchk, sizeof(double) * (nbx + 1));
             e.alloc(&bs, sizeof(double) * 14 * nblk);
@@ -114,12 +112,12 @@ struct BasicRunner {
     }
     void release()
     {
-        for (void* q : {(void*)f6, (void*)f1, (void*)S6, (void*)S12, (void*)Eh, (void*)psum, (void*)psum2, (void*)pfin, (void*)pchk,
+        for (void* q : {(void*)f6, (void*)f1, (void*)S6, (void*)S12, (void*)Eh, (void*)psum, (void*)pfin, (void*)pchk,
                         (void*)bs, (void*)mat, (void*)ctl, (void*)f6s, (void*)f1s, (void*)S6s, (void*)S12s, (void*)Ehs})
             if (q) (void)hipFree(q);
         if (hs) (void)hipHostFree(hs);
         hs = nullptr;
-        f6 = f1 = psum = psum2 = pfin = pchk = bs = mat = nullptr;
+        f6 = f1 = psum = pfin = pchk = bs = mat = nullptr;
         S6 = S12 = Eh = nullptr;
         f6s = f1s = nullptr;
         S6s = S12s = Ehs = nullptr;
@@ -193,17 +191,8 @@ struct BasicRunner {
     BPtr<double> bptr() { return bptr_t<double>(); }
     Ptr<double> yptr() { return yptr_t<double>(); }
 
-    // the per-solve sums of the z pass (two launches, fixed order) and the
-    // increment/iteration bookkeeping that follows them
-    template <int MODE>
-    void bfin1(const Geo& g)
-    {
-        hipLaunchKernelGGL(k_bsum_parts<0>, dim3(BSPLIT, NBSUM, 1), dim3(256), 0, e.st, g, ctl, psum, psum2);
-        hipLaunchKernelGGL((k_bfin1<MODE>), dim3(1), dim3(FTHREADS), 0, e.st, g, ctl, psum2);
-    }
-
-    // one stage: z pass, sums and updateE, y pass, x pass, stop rule, y pass; the
-    // restart stage is a start stage (strain from HBM) that keeps itNo.  A
+    // one stage: z pass, y pass with the sums and updateE beside it, x pass, y
+    // pass with the stop rule beside it; the restart stage is a start stage (strain from HBM) that keeps itNo.  A
     // start stage transforms [sigma | eps] and writes S6 buffer 0 (par = 1);
     // an iteration reads S6 buffer par, transforms sigma only (the x pass
     // keeps eps^ in Eh) and writes buffer 1 - par.
@@ -219,22 +208,18 @@ struct BasicRunner {
         if (fast) bfast::launch_z<T>(beh, zm, g, bp, st, lin);
         else if constexpr (sizeof(T) == 8)
             bflex::launch_z(beh, zm, g, bp, st, lin);
-        if (mode == BMODE_START) bfin1<BMODE_START>(g);
-        else if (mode == BMODE_RESTART)
-            bfin1<BMODE_RESTART>(g);
-        else bfin1<BMODE_ITER>(g);
+        const BFin f1{1, mode, g.nbz, g.invN, psum, nullptr};
+        const BFin f2{2, mode, g.nbx, g.invN, pchk, iter ? hs : nullptr};
         if (fast) {
-            if (iter) bfast::launch_y6_fwd<T>(gf6, yp, st);
-            else bfast::launch_y12<T>(gf, yp, st);
+            if (iter) bfast::launch_y6_fwd<T>(gf6, yp, f1, st);
+            else bfast::launch_y12<T>(gf, yp, f1, st);
             bfast::launch_x<T>(gf, bp, st, iter);
+            bfast::launch_y6<T>(gf6, yp, f2, st);
         } else if constexpr (sizeof(T) == 8) {
-            flex::launch_y<T>(-1, BUF_K, 0, g, yp, st);
+            bflex::launch_y(-1, BUF_K, g, yp, f1, st);
             bflex::launch_x(g, bp, st, iter);
+            bflex::launch_y(1, BUF_MAIN, g6, yp, f2, st);
         }
-        hipLaunchKernelGGL((k_bfin2<0>), dim3(1), dim3(FTHREADS), 0, st, g, ctl, pchk, iter ? hs : nullptr);
-        if (fast) bfast::launch_y6<T>(gf6, yp, st);
-        else if constexpr (sizeof(T) == 8)
-            flex::launch_y<T>(1, BUF_MAIN, 0, g6, yp, st);
     }
 
     // the fields and state of the increment's last iterate on the FP64 path,

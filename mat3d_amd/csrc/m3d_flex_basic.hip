@@ -281,6 +281,21 @@ __global__ void __launch_bounds__(NT) k_xb(Geo g, BPtr<T> p)
     flex::store_tile<T, NT>(sl, p.S6w + ((long long)y * g.Nzh + kz0) * 6, (long long)g.Ny * g.Nzh * 6, g.Nx, w6);
 }
 
+// ------------------------------------------------------------------ y pass
+// flex::k_y with the finaliser f as its first workgroup
+template <int DIR, int NT>
+__global__ void __launch_bounds__(NT) k_yb(Geo g, Ptr<T> p, int which, BFin f)
+{
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    __shared__ double red[NT / 64][NBSUM];
+    if (blockIdx.x == 0) {
+        bfin_block(p.ctl[0], f, red);
+        return;
+    }
+    cx<T>* sl = reinterpret_cast<cx<T>*>(smem_raw);
+    flex::y_tile<T, DIR, NT>(g, p, which, fast::xcd_remap(blockIdx.x - 1, gridDim.x - 1), sl, sl + (size_t)g.Ny * g.TKy * g.C);
+}
+
 // ---------------------------------------------------------------- planning
 namespace {
 
@@ -299,15 +314,15 @@ int even(int n, int most)
     return (n + parts - 1) / parts;
 }
 
-template <typename K>
-void go(K* k, int blocks, int nt, size_t sm, const Geo& g, const BPtr<T>& p, hipStream_t st)
+template <typename K, typename... A>
+void go(K* k, int blocks, int nt, size_t sm, hipStream_t st, const A&... args)
 {
     if (sm > 65536) {
         const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(k),
                                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)sm);
         if (e != hipSuccess) throw std::runtime_error(std::string("LDS size: ") + hipGetErrorString(e));
     }
-    hipLaunchKernelGGL(k, dim3(blocks), dim3(nt), sm, st, g, p);
+    hipLaunchKernelGGL(k, dim3(blocks), dim3(nt), sm, st, args...);
 }
 
 template <int BEH, int MODE, bool LIN>
@@ -315,8 +330,8 @@ void z_at(const Geo& g, const BPtr<T>& p, hipStream_t st)
 {
     constexpr int HC = MODE == BMODE_START ? 6 : 3;
     const size_t W = (size_t)(g.TY * HC) | 1;
-    if (z_rows(g.Nz, 2 * HC, NT0) >= 1) go(&k_zb<BEH, MODE, LIN, NT0>, g.nbz, NT0, g.Nz * (W + 1) * sizeof(cx<T>), g, p, st);
-    else go(&k_zb<BEH, MODE, LIN, NT1>, g.nbz, NT1, g.Nz * W * sizeof(cx<T>), g, p, st);
+    if (z_rows(g.Nz, 2 * HC, NT0) >= 1) go(&k_zb<BEH, MODE, LIN, NT0>, g.nbz, NT0, g.Nz * (W + 1) * sizeof(cx<T>), st, g, p);
+    else go(&k_zb<BEH, MODE, LIN, NT1>, g.nbz, NT1, g.Nz * W * sizeof(cx<T>), st, g, p);
 }
 
 template <int BEH, bool LIN>
@@ -349,17 +364,32 @@ void launch_z(int beh, int mode, const Geo& g, const BPtr<T>& p, hipStream_t st,
     else z_beh<BEH_ED, false>(mode, g, p, st);
 }
 
+void launch_y(int dir, int which, const Geo& g, const Ptr<T>& p, const BFin& f, hipStream_t st)
+{
+    const long tile = (long)g.Ny * g.TKy * g.C;
+    const bool lg = tile > (long)flex::ept<T, NT0>() * NT0;
+    const size_t sm = (size_t)(tile + (lg ? 0 : g.Ny)) * sizeof(cx<T>);
+    const int blocks = g.Nx * g.nky + 1;
+    if (dir < 0) {
+        if (lg) go(&k_yb<-1, NT1>, blocks, NT1, sm, st, g, p, which, f);
+        else go(&k_yb<-1, NT0>, blocks, NT0, sm, st, g, p, which, f);
+    } else {
+        if (lg) go(&k_yb<1, NT1>, blocks, NT1, sm, st, g, p, which, f);
+        else go(&k_yb<1, NT0>, blocks, NT0, sm, st, g, p, which, f);
+    }
+}
+
 void launch_x(const Geo& g, const BPtr<T>& p, hipStream_t st, bool e6)
 {
     const size_t tile = (size_t)g.Nx * g.TKx * g.C;
     const bool lg = x_cols(g.Nx, g.C, NT0) < 1;
     const size_t sm = (tile + (lg ? 0 : g.Nx)) * sizeof(cx<T>);
     if (e6) {
-        if (lg) go(&k_xb<true, NT1>, g.nbx, NT1, sm, g, p, st);
-        else go(&k_xb<true, NT0>, g.nbx, NT0, sm, g, p, st);
+        if (lg) go(&k_xb<true, NT1>, g.nbx, NT1, sm, st, g, p);
+        else go(&k_xb<true, NT0>, g.nbx, NT0, sm, st, g, p);
     } else {
-        if (lg) go(&k_xb<false, NT1>, g.nbx, NT1, sm, g, p, st);
-        else go(&k_xb<false, NT0>, g.nbx, NT0, sm, g, p, st);
+        if (lg) go(&k_xb<false, NT1>, g.nbx, NT1, sm, st, g, p);
+        else go(&k_xb<false, NT0>, g.nbx, NT0, sm, st, g, p);
     }
 }
 
