@@ -2,21 +2,25 @@
 // the basic scheme on complex 2D fields [E11, E22, E12] (tensor shear) with
 // a fixed 25 iterations per runAnalysis.
 //
-// Per iteration (four launches):
-//   polar : eps = t / xy of the previous iteration (FFTBCKWRD_epsilon
-//           :143-148); sigma = C(phase) eps (multipCx, :96-106); tau =
-//           sigma - C0 eps (:240)
-//   y     : forward FFT along y of the three interleaved components (p3)
-//   x     : forward FFT along x, then t = -G(xi) t with the reference's
-//           6-entry Green operator per frequency (setGF :53-93, recomputed
-//           here; x > (Nx-1)/2 maps to -(Ny - x) as in the reference), DC =
-//           E xy (multiplyGF :114-141), then the backward FFT along x
-//   y     : backward FFT along y (p4)
+// Per iteration (two launches):
+//   row : one x row in LDS: backward FFT along y (p4), eps = t / xy of the
+//         previous iteration (FFTBCKWRD_epsilon :143-148); sigma = C(phase) eps
+//         (multipCx, :96-106); tau = sigma - C0 eps (:240); forward FFT along y
+//         of the three interleaved components (p3).  The first row pass reads
+//         eps, the last one ends after eps; sigma is stored by the last
+//         iteration only (nothing else reads it)
+//   x   : forward FFT along x, then t = -G(xi) t with the reference's
+//         6-entry Green operator per frequency (setGF :53-93, recomputed
+//         here; x > (Nx-1)/2 maps to -(Ny - x) as in the reference), DC =
+//         E xy (multiplyGF :114-141), then the backward FFT along x
 // convergenceCheck (:150-187) only prints, and its sum reads past the two-entry
 // frequency vector; its iteration counter is kept, its transform is not.
-// The 1D transforms are the y/x passes of m3d_fast.hpp on a three-component
-// view: y lines are rows of one x plane (3 values apart), x lines are rows
-// Ny*3 values apart with the y index in the role of the contiguous kz tile.
+// The x pass is that of m3d_fast.hpp on a three-component view: x lines are
+// rows Ny*3 values apart with the y index in the role of the contiguous kz tile.
+// The 75 iterations of a homogenization are a chain of dependent launches, bound
+// by their latency up to 512^2: with four launches per iteration (62 us) and the
+// means taken on the host from 75 MB of copied fields a 512^2 homogenization
+// took 11.7 ms, with two launches and row sums taken on the device 2.7 ms.
 #include "m3d_engine.hpp"
 
 #include <cstring>
@@ -35,36 +39,92 @@ struct Comp3 {
     static __device__ void green(const Geo& g, const Ctl& ctl, const T* prm, int kx, int, int kz, cx<T>* v);
 };
 
-constexpr int NT = 256;
+// threads of the row pass and of the x pass (128, 192 and 512 within 3-10%)
+constexpr int NTR = 256, NTX = 256;
 
 struct Mat {
     double Cm[9], Ci[9], C0[9];
     double la0, mu0;
 };
 
-// from_t: the previous iteration's strain is still the unscaled inverse
-// transform in t; eps = t / xy is stored first (the scaling step of the
-// previous iteration, done here to save a launch)
-__global__ void k_polar(const uint8_t* ph, Mat m, cx<double>* eps, cx<double>* sig, cx<double>* t, long long xy,
-                        int from_t)
+// FIRST: eps is read (no backward transform), LAST: ends after storing eps.
+// psum: the row's sums of the real parts, [6][Nx] (eps by the LAST pass, sigma
+// by the pass that stores it)
+template <int L, bool FIRST, bool LAST>
+__global__ void __launch_bounds__(NTR) k_row(const uint8_t* ph, Mat m, cx<double>* eps, cx<double>* sig, cx<double>* t,
+                                             const cx<double>* twg, double xy, int store_sig, double* psum)
 {
+    __shared__ __align__(16) cx<double> sl[3 * L];
+    __shared__ cx<double> tw[L];
+    __shared__ double red[NTR / 64];
+    const int x = blockIdx.x, nx = gridDim.x;
+    const long long row = (long long)x * L;
+    const cx<double>* src = (FIRST ? eps : t) + 3 * row;
+    constexpr int PER = (3 * L + NTR - 1) / NTR;
+    {
+        fast::vd2 r[PER];
+#pragma unroll
+        for (int i = 0; i < PER; ++i)
+            if ((3 * L) % NTR == 0 || (int)threadIdx.x + i * NTR < 3 * L)
+                r[i] = *reinterpret_cast<const fast::vd2*>(src + threadIdx.x + i * NTR);
+        for (int i = threadIdx.x; i < L; i += NTR) tw[i] = twg[i];
+#pragma unroll
+        for (int i = 0; i < PER; ++i)
+            if ((3 * L) % NTR == 0 || (int)threadIdx.x + i * NTR < 3 * L)
+                *reinterpret_cast<fast::vd2*>(sl + threadIdx.x + i * NTR) = r[i];
+    }
+    __syncthreads();
+    if constexpr (!FIRST) fast::fft<double, L, 3, NTR, 1, 1>(sl, tw);
+    double se[3] = {0, 0, 0}, ss[3] = {0, 0, 0};
+    for (int y = threadIdx.x; y < L; y += NTR) {
 #pragma clang fp contract(off)
-    const long long s0 = blockIdx.x * (long long)blockDim.x + threadIdx.x, st = (long long)gridDim.x * blockDim.x;
-    for (long long i = s0; i < xy; i += st) {
-        const double* C = ph[i] ? m.Cm : m.Ci;
-        if (from_t) {
-            const double n = (double)xy;
-            for (int c = 0; c < 3; ++c) eps[3 * i + c] = cx<double>{t[3 * i + c].re / n, t[3 * i + c].im / n};
+        cx<double> e[3];
+        for (int c = 0; c < 3; ++c) {
+            e[c] = sl[3 * y + c];
+            if (!FIRST) e[c] = cx<double>{e[c].re / xy, e[c].im / xy};
         }
-        const cx<double> e0 = eps[3 * i], e1 = eps[3 * i + 1], e2 = eps[3 * i + 2];
+        if constexpr (LAST) {
+            for (int c = 0; c < 3; ++c) {
+                eps[3 * (row + y) + c] = e[c];
+                se[c] += e[c].re;
+            }
+            continue;
+        }
+        const double* C = ph[row + y] ? m.Cm : m.Ci;
         for (int r = 0; r < 3; ++r) {
-            const cx<double> sg{(C[3 * r] * e0.re + C[3 * r + 1] * e1.re) + C[3 * r + 2] * e2.re,
-                                (C[3 * r] * e0.im + C[3 * r + 1] * e1.im) + C[3 * r + 2] * e2.im};
-            const cx<double> c0{(m.C0[3 * r] * e0.re + m.C0[3 * r + 1] * e1.re) + m.C0[3 * r + 2] * e2.re,
-                                (m.C0[3 * r] * e0.im + m.C0[3 * r + 1] * e1.im) + m.C0[3 * r + 2] * e2.im};
-            sig[3 * i + r] = sg;
-            t[3 * i + r] = cx<double>{sg.re - c0.re, sg.im - c0.im};
+            const cx<double> sg{(C[3 * r] * e[0].re + C[3 * r + 1] * e[1].re) + C[3 * r + 2] * e[2].re,
+                                (C[3 * r] * e[0].im + C[3 * r + 1] * e[1].im) + C[3 * r + 2] * e[2].im};
+            const cx<double> c0{(m.C0[3 * r] * e[0].re + m.C0[3 * r + 1] * e[1].re) + m.C0[3 * r + 2] * e[2].re,
+                                (m.C0[3 * r] * e[0].im + m.C0[3 * r + 1] * e[1].im) + m.C0[3 * r + 2] * e[2].im};
+            if (store_sig) {
+                sig[3 * (row + y) + r] = sg;
+                ss[r] += sg.re;
+            }
+            sl[3 * y + r] = cx<double>{sg.re - c0.re, sg.im - c0.im};
         }
+    }
+    if (LAST || store_sig) {
+        for (int c = 0; c < 3; ++c) {
+            const double v = block_sum(LAST ? se[c] : ss[c], red);
+            if (threadIdx.x == 0) psum[(long long)(LAST ? c : 3 + c) * nx + x] = v;
+        }
+    }
+    if constexpr (LAST) return;
+    __syncthreads();
+    fast::fft<double, L, 3, NTR, -1, 1>(sl, tw);
+    cx<double>* dst = t + 3 * row;
+#pragma unroll
+    for (int i = 0; i < PER; ++i)
+        if ((3 * L) % NTR == 0 || (int)threadIdx.x + i * NTR < 3 * L) dst[threadIdx.x + i * NTR] = sl[threadIdx.x + i * NTR];
+}
+
+// setLoad: eps = E at every point
+__global__ void k_fill_eps(cx<double>* eps, cx<double> e0, cx<double> e1, cx<double> e2, long long xy)
+{
+    for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < xy; i += (long long)gridDim.x * blockDim.x) {
+        eps[3 * i] = e0;
+        eps[3 * i + 1] = e1;
+        eps[3 * i + 2] = e2;
     }
 }
 
@@ -113,12 +173,6 @@ __device__ void Comp3::green(const Geo& g, const Ctl& ctl, const T* prm, int kx,
 
 static_assert(fast::has_green_hook<Comp3>::value, "the 2D Green step must replace the 3D one in the x pass");
 
-__global__ void k_scale(const cx<double>* t, cx<double>* eps, long long n3, double xy)
-{
-    const long long s0 = blockIdx.x * (long long)blockDim.x + threadIdx.x, st = (long long)gridDim.x * blockDim.x;
-    for (long long k = s0; k < n3; k += st) eps[k] = cx<double>{t[k].re / xy, t[k].im / xy};
-}
-
 inline bool fast_len(int L)
 {
     return L == 32 || L == 48 || L == 64 || L == 96 || L == 128 || L == 192 || L == 256 || L == 512;
@@ -134,12 +188,12 @@ struct Solver {
     cx<double>*twx = nullptr, *twy = nullptr;
     double* dprm = nullptr; // {la0, mu0} for the Green step
     int* drve = nullptr;    // {0}: the one solve's parameter row
-    Geo gy{}, gx1{};
+    double* psum = nullptr; // [6][Nx] row sums of the real parts of eps and sigma
+    Geo gx1{};
     Mat m{};
     cx<double> E[3] = {{0, 0}, {0, 0}, {0, 0}};
     bool have_mat = false;
     int itNo = 0;
-    int nb = 1024;
 
     template <typename P>
     void alloc(P** p, size_t bytes)
@@ -165,6 +219,7 @@ struct Solver {
         alloc(&ctl, sizeof(Ctl));
         alloc(&dprm, sizeof(double) * 2);
         alloc(&drve, sizeof(int));
+        alloc(&psum, sizeof(double) * 6 * nx);
         HCHK(hipMemset(drve, 0, sizeof(int)));
         HCHK(hipMemset(eps, 0, sizeof(cx<double>) * 3 * xy));
         HCHK(hipMemset(sig, 0, sizeof(cx<double>) * 3 * xy));
@@ -174,51 +229,37 @@ struct Solver {
         alloc(&twy, sizeof(cx<double>) * ny);
         HCHK(hipMemcpy(twx, tx.data(), sizeof(cx<double>) * nx, hipMemcpyHostToDevice));
         HCHK(hipMemcpy(twy, ty.data(), sizeof(cx<double>) * ny, hipMemcpyHostToDevice));
-        // y lines: one tile per x plane (rows y at stride 3, one "kz" column of
-        // 3 components); x lines: rows x at stride Ny*3, the Ny points of a row
-        // in the role of the kz tile
-        std::memset(&gy, 0, sizeof gy);
-        gy.Nx = nx; gy.Ny = ny; gy.Nz = 1; gy.Nzh = 1; gy.C = 3; gy.nsolve = 1;
-        gy.sy = 3; gy.sxa = (long long)ny * 3; gy.sxb = 0; gy.lxb = 0; gy.xbm = 0;
         // x lines with the Green step: the grid as nx x 1 x ny, rows x at
         // stride ny*3, the y points in the role of the kz tile
-        gx1 = gy;
-        gx1.Nx = nx; gx1.Ny = 1; gx1.Nzh = ny;
+        std::memset(&gx1, 0, sizeof gx1);
+        gx1.Nx = nx; gx1.Ny = 1; gx1.Nz = 1; gx1.Nzh = ny; gx1.C = 3; gx1.nsolve = 1;
         gx1.sy = (long long)ny * 3; gx1.sxa = (long long)ny * 3; gx1.sxb = 0; gx1.lxb = 0; gx1.xbm = 0;
     }
 
     ~Solver()
     {
         if (st) (void)hipStreamSynchronize(st);
-        for (void* p : {(void*)eps, (void*)sig, (void*)t, (void*)ph, (void*)ctl, (void*)dprm, (void*)drve, (void*)twx,
-                        (void*)twy})
+        for (void* p : {(void*)eps, (void*)sig, (void*)t, (void*)ph, (void*)ctl, (void*)dprm, (void*)drve, (void*)psum,
+                        (void*)twx, (void*)twy})
             if (p) (void)hipFree(p);
         if (st) (void)hipStreamDestroy(st);
     }
 
-    template <int L, int TK, int DIR>
-    bool pass_at(const Geo& g, const cx<double>* tw)
+    template <int L, bool FIRST, bool LAST>
+    bool row_at(int store_sig)
     {
-        if (g.Ny != L) return false;
-        const int nkt = (g.Nzh + TK - 1) / TK;
-        const size_t sm = ((size_t)L * TK * 3 + L) * sizeof(cx<double>);
-        Ptr<double> p;
-        std::memset(&p, 0, sizeof p);
-        p.S = t;
-        p.K = t;
-        p.twy = tw;
-        p.ctl = ctl;
-        hipLaunchKernelGGL((fast::kxy<double, Comp3, 0, DIR, BUF_MAIN, L, TK, NT>), dim3(g.Nx * nkt), dim3(NT), sm, st, g,
-                           p, (const double*)nullptr);
+        if (Ny != L) return false;
+        hipLaunchKernelGGL((k_row<L, FIRST, LAST>), dim3(Nx), dim3(NTR), 0, st, ph, m, eps, sig, t, twy, (double)xy, store_sig,
+                           psum);
         return true;
     }
-    // y pass: one kz column (TK = 1); x pass: kz tiles of the library's width
-    template <int DIR>
-    void ypass()
+    template <bool FIRST, bool LAST>
+    void row(int store_sig)
     {
-        if (!(pass_at<512, 1, DIR>(gy, twy) || pass_at<256, 1, DIR>(gy, twy) || pass_at<192, 1, DIR>(gy, twy) ||
-              pass_at<128, 1, DIR>(gy, twy) || pass_at<96, 1, DIR>(gy, twy) || pass_at<64, 1, DIR>(gy, twy) ||
-              pass_at<48, 1, DIR>(gy, twy) || pass_at<32, 1, DIR>(gy, twy)))
+        if (!(row_at<512, FIRST, LAST>(store_sig) || row_at<256, FIRST, LAST>(store_sig) ||
+              row_at<192, FIRST, LAST>(store_sig) || row_at<128, FIRST, LAST>(store_sig) ||
+              row_at<96, FIRST, LAST>(store_sig) || row_at<64, FIRST, LAST>(store_sig) ||
+              row_at<48, FIRST, LAST>(store_sig) || row_at<32, FIRST, LAST>(store_sig)))
             throw ArgError{M3D_ERR_UNSUPPORTED, "FFT_Analysis2D: no y kernel"};
     }
     // x lines: forward FFT, the Green step (Comp3::green), inverse FFT in one
@@ -227,7 +268,9 @@ struct Solver {
     bool xg_at()
     {
         if (gx1.Nx != L) return false;
-        constexpr int TK = fast::xtile<double>(L, 3);
+        // one y point per tile: as many workgroups as rows (tiles of the 3D
+        // width left 16 workgroups for a 128^2 plate)
+        constexpr int TK = 1;
         const int nkt = (gx1.Nzh + TK - 1) / TK;
         const size_t sm = ((size_t)L * TK * 3 + L) * sizeof(cx<double>);
         if (sm > 65536) throw ArgError{M3D_ERR_UNSUPPORTED, "FFT_Analysis2D: x tile too large"};
@@ -238,7 +281,7 @@ struct Solver {
         p.twx = twx;
         p.ctl = ctl;
         p.rve_of = drve;
-        hipLaunchKernelGGL((fast::kxy<double, Comp3, 1, -1, BUF_MAIN, L, TK>), dim3(nkt), dim3(NT), sm, st, gx1, p,
+        hipLaunchKernelGGL((fast::kxy<double, Comp3, 1, -1, BUF_MAIN, L, TK, NTX>), dim3(nkt), dim3(NTX), sm, st, gx1, p,
                            (const double*)dprm);
         return true;
     }
@@ -273,25 +316,29 @@ struct Solver {
         have_mat = true;
     }
 
-    // runAnalysis, :232-246
-    void run()
+    // runAnalysis, :232-246, without waiting for it; e_ri: the load, alive
+    // until the stream is synchronised
+    void run_async(const double* e_ri)
     {
         if (!have_mat) throw ArgError{M3D_ERR_STATE, "runAnalysis: material() first"};
+        HCHK(hipMemcpyAsync(reinterpret_cast<char*>(ctl) + offsetof(Ctl, E), e_ri, 6 * sizeof(double), hipMemcpyHostToDevice, st));
+        for (int it = 0; it < 25; ++it) {
+            if (it == 0) row<true, false>(0);
+            else row<false, false>(it == 24);
+            xgreen();
+            itNo += 1;
+        }
+        row<false, true>(0);
+        HCHK(hipGetLastError());
+    }
+    void run()
+    {
         double e_ri[6];
         for (int c = 0; c < 3; ++c) {
             e_ri[2 * c] = E[c].re;
             e_ri[2 * c + 1] = E[c].im;
         }
-        HCHK(hipMemcpy(reinterpret_cast<char*>(ctl) + offsetof(Ctl, E), e_ri, sizeof e_ri, hipMemcpyHostToDevice));
-        for (int it = 0; it < 25; ++it) {
-            hipLaunchKernelGGL(k_polar, dim3(nb), dim3(NT), 0, st, ph, m, eps, sig, t, xy, it > 0 ? 1 : 0);
-            ypass<-1>();
-            xgreen();
-            ypass<1>();
-            itNo += 1;
-        }
-        hipLaunchKernelGGL(k_scale, dim3(nb), dim3(NT), 0, st, t, eps, 3 * xy, (double)xy);
-        HCHK(hipGetLastError());
+        run_async(e_ri);
         HCHK(hipStreamSynchronize(st));
     }
 };
@@ -409,10 +456,8 @@ int m3d_2d_set_load(m3d_2d* h, const double* E_ri)
         if (!E_ri) throw ArgError{M3D_ERR_ARG, "setLoad: null argument"};
         p2::Solver& s = *h->s;
         for (int c = 0; c < 3; ++c) s.E[c] = cx<double>{E_ri[2 * c], E_ri[2 * c + 1]};
-        std::vector<cx<double>> e((size_t)(3 * s.xy));
-        for (long long i = 0; i < s.xy; ++i)
-            for (int c = 0; c < 3; ++c) e[(size_t)(3 * i + c)] = s.E[c];
-        HCHK(hipMemcpy(s.eps, e.data(), sizeof(cx<double>) * e.size(), hipMemcpyHostToDevice));
+        hipLaunchKernelGGL(p2::k_fill_eps, dim3(256), dim3(256), 0, s.st, s.eps, s.E[0], s.E[1], s.E[2], s.xy);
+        HCHK(hipGetLastError());
         return M3D_OK;
     });
 }
@@ -430,24 +475,31 @@ int m3d_2d_homogenization(m3d_2d* h, double* CHomo, double* epHomo, double* sigH
 {
     return guarded(h, [&]() {
         p2::Solver& s = *h->s;
-        double ep[9], sg[9];
-        std::vector<cx<double>> e((size_t)(3 * s.xy)), g((size_t)(3 * s.xy));
+        double ep[9], sg[9], loads[3][6];
+        std::vector<double> sums((size_t)3 * 6 * s.Nx);
+        // the three load cases follow each other on the device; their row sums
+        // come back together
         for (int w = 0; w < 3; ++w) {
-            for (int c = 0; c < 3; ++c) s.E[c] = cx<double>{c == w ? 0.005 : 0.0, 0.0};
-            s.run();
-            HCHK(hipMemcpy(e.data(), s.eps, sizeof(cx<double>) * e.size(), hipMemcpyDeviceToHost));
-            HCHK(hipMemcpy(g.data(), s.sig, sizeof(cx<double>) * g.size(), hipMemcpyDeviceToHost));
-            double se[3] = {0, 0, 0}, ss[3] = {0, 0, 0};
-            for (long long i = 0; i < s.xy; ++i)
-                for (int c = 0; c < 3; ++c) {
-                    se[c] += e[(size_t)(3 * i + c)].re;
-                    ss[c] += g[(size_t)(3 * i + c)].re;
-                }
             for (int c = 0; c < 3; ++c) {
-                ep[w + 3 * c] = se[c] / (double)s.xy;
-                sg[c + 3 * w] = ss[c] / (double)s.xy;
+                s.E[c] = cx<double>{c == w ? 0.005 : 0.0, 0.0};
+                loads[w][2 * c] = s.E[c].re;
+                loads[w][2 * c + 1] = 0.0;
             }
+            s.run_async(loads[w]);
+            HCHK(hipMemcpyAsync(sums.data() + (size_t)w * 6 * s.Nx, s.psum, sizeof(double) * 6 * s.Nx, hipMemcpyDeviceToHost,
+                                s.st));
         }
+        HCHK(hipStreamSynchronize(s.st));
+        for (int w = 0; w < 3; ++w)
+            for (int c = 0; c < 3; ++c) {
+                double se = 0, ss = 0;
+                for (int x = 0; x < s.Nx; ++x) {
+                    se += sums[((size_t)w * 6 + c) * s.Nx + x];
+                    ss += sums[((size_t)w * 6 + 3 + c) * s.Nx + x];
+                }
+                ep[w + 3 * c] = se / (double)s.xy;
+                sg[c + 3 * w] = ss / (double)s.xy;
+            }
         double inv[9];
         if (!inv3(ep, inv)) throw ArgError{M3D_ERR_NUMERIC, "homogenization: singular epHomo"};
         double C[9];
