@@ -286,17 +286,17 @@ __global__ void __launch_bounds__(ZNT) M3D_BZ_ATTR kzb(Geo g, BPtr<T> p)
 //   E6 = true (after an ITER z pass): sigma^ comes from S12 with 6
 //     components per kz (LDS row kx: W = 6 TK columns, kzl*6 + c); eps^ is
 //     read from Eh, where the previous x pass left it already x-transformed,
-//     by the thread that applies the Green step to it (L*TK <= XNT: one
+//     by the thread that applies the Green step to it (L*TK <= threads: one
 //     frequency per thread), issued with the sigma^ loads so that it arrives
 //     during the forward FFT.
 // Both write the new eps^ (unnormalised, before the inverse x FFT) to Eh,
 // one contiguous [kx][kzl][c] block per tile, for the next iteration.
 template <typename T, int L, int TK, bool E6>
-__global__ void __launch_bounds__(XNT) M3D_BX_ATTR kxb(Geo g, BPtr<T> p)
+__global__ void __launch_bounds__(xthreads(L)) M3D_BX_ATTR kxb(Geo g, BPtr<T> p)
 {
     constexpr int C = E6 ? 6 : 12; // LDS columns per kz
     constexpr int W = TK * C;
-    constexpr int NT = XNT;
+    constexpr int NT = xthreads(L);
     extern __shared__ __align__(16) unsigned char smem_raw[];
     __shared__ double red[NT / 64];
     cx<T>* sl = reinterpret_cast<cx<T>*>(smem_raw);
@@ -476,7 +476,7 @@ bool x_at(const Geo& g, const BPtr<T>& p, hipStream_t st)
     if (sm > 65536)
         (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&kxb<T, L, TK, E6>),
                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)sm);
-    hipLaunchKernelGGL((kxb<T, L, TK, E6>), dim3(g.nbx), dim3(XNT), sm, st, g, p);
+    hipLaunchKernelGGL((kxb<T, L, TK, E6>), dim3(g.nbx), dim3(xthreads(L)), sm, st, g, p);
     return true;
 }
 

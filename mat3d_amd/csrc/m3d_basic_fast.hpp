@@ -19,9 +19,6 @@ namespace bfast {
 #ifndef M3D_BZ_PAD
 #define M3D_BZ_PAD 0 // complex values of padding per LDS row of the z pass
 #endif
-#ifndef M3D_BX_THREADS
-#define M3D_BX_THREADS 512
-#endif
 #ifndef M3D_BX_TILE
 #define M3D_BX_TILE 6144
 #endif
@@ -44,7 +41,11 @@ namespace bfast {
 #define M3D_BX_ATTR
 #endif
 constexpr int ZNT = M3D_BZ_THREADS; // threads of the z pass
-constexpr int XNT = M3D_BX_THREADS; // threads of the x pass
+// x pass: lines of up to 128 points on half tiles of 256 threads (two more
+// workgroups per CU to overlap), longer ones on full tiles of 512.  Measured per
+// J2 load path, half against full: 32^3 15.3 / 16.1 ms, 48^3 25.2 / 25.7, 64^3
+// 49.9 / 50.9, 96^3 82.8 / 91.7, 128^3 190 / 193, 192^3 670 / 648.
+constexpr int xthreads(int L) { return L <= 128 ? 256 : 512; }
 
 // z tile: TY lines (y) of 12 components each, TY*12*LZ <= M3D_BZ_TILE complex
 constexpr int zlines(int LZ, int Ny)
@@ -53,10 +54,11 @@ constexpr int zlines(int LZ, int Ny)
     while (ty < 8 && (ty * 2) * 12 * LZ <= M3D_BZ_TILE && Ny % (ty * 2) == 0) ty *= 2;
     return ty;
 }
-// x tile: TK kz values of 12 components (TK * L <= M3D_BX_TILE / 12)
+// x tile: TK kz values of 12 components (TK * L <= M3D_BX_TILE / 12, half of it
+// for short lines)
 constexpr int xtile(int L)
 {
-    const int tk = M3D_BX_TILE / (12 * L);
+    const int tk = (L <= 128 ? M3D_BX_TILE / 2 : M3D_BX_TILE) / (12 * L);
     return tk < 1 ? 1 : tk;
 }
 // y tiles (the generic fast y pass with 12 / 6 components)

@@ -107,12 +107,31 @@ constexpr int zlines(int LZ, int C, int Ny)
 #ifndef M3D_YTILE
 #define M3D_YTILE 6144
 #endif
+// kz values of a tile of ``budget`` values.  Lines of up to 48 points: their
+// grids leave one or two workgroups per CU, so the longest workgroup is what a
+// launch waits for.  FP32 tiles share Nz/2+1 kz (taken as for a cube) evenly:
+// 13 + 12 instead of 21 + 4 at 48, and one tile of 17 instead of LDS for 32 at
+// 32; FP64 tiles take half the budget (at 32: 8, 8, 1 instead of 16, 1).
+// Before -> after per homogenization: 32^3 FP64 0.96 -> 0.91 ms, FP32 1.59 ->
+// 1.53; 48^3 FP64 2.75 -> 2.51, FP32 2.88 -> 2.67; batch of 16 x 32^3 and 8 x 48^3
+// FP64 11.4 -> 10.5, FP32 8.9 -> 8.2.  Even FP64 tiles (6, 6, 5) are 2% slower at
+// 32.  Longer lines keep the budget's tile: halved tiles are 1-2% slower at 64
+// and 128, even ones 7% at 64 FP64 (11 kz, no shift for the division by it).
+template <typename T>
+constexpr int ktile(int budget, int L, int C)
+{
+    const int tk = budget / (C * L);
+    if (L > 48) return tk < 1 ? 1 : tk;
+    const int n = L / 2 + 1;
+    if (sizeof(T) == 8) return tk / 2 < n ? tk / 2 : n;
+    const int nt = (n + tk - 1) / tk;
+    return (n + nt - 1) / nt;
+}
 template <typename T>
 constexpr int xytile(int L, int C)
 {
     int budget = sizeof(T) == 4 ? M3D_YTILE : M3D_YTILE / 2;
-    int tk = budget / (C * L);
-    return tk < 1 ? 1 : tk;
+    return ktile<T>(budget, L, C);
 }
 // x passes: complex values per tile (FP32; FP64 half); the x lines are one
 // (y, kz) row apart, Ny*Nzh*C values, so wider kz tiles amortise each row visit
@@ -123,8 +142,7 @@ template <typename T>
 constexpr int xtile(int L, int C)
 {
     int budget = sizeof(T) == 4 ? M3D_XTILE : M3D_XTILE / 2;
-    int tk = budget / (C * L);
-    return tk < 1 ? 1 : tk;
+    return ktile<T>(budget, L, C);
 }
 // x pass of the equilibrium check (FP32): narrower kz tiles, so more
 // workgroups share a CU's LDS while the tile is read (the pass only reads)
@@ -135,16 +153,14 @@ template <typename T>
 constexpr int xctile(int L, int C)
 {
     int budget = sizeof(T) == 4 ? M3D_XCTILE : M3D_XTILE / 2;
-    int tk = budget / (C * L);
-    return tk < 1 ? 1 : tk;
+    return ktile<T>(budget, L, C);
 }
 // the autotuner's wide alternative for the x pass with the Green step (1.5x)
 template <typename T>
 constexpr int xtile_wide(int L, int C)
 {
     int budget = (sizeof(T) == 4 ? M3D_XTILE : M3D_XTILE / 2) * 3 / 2;
-    int tk = budget / (C * L);
-    return tk < 1 ? 1 : tk;
+    return ktile<T>(budget, L, C);
 }
 constexpr int ZNT = 256;
 
