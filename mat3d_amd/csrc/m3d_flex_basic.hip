@@ -314,6 +314,14 @@ int even(int n, int most)
     return (n + parts - 1) / parts;
 }
 
+// kz values of an x or y tile that leave 384 workgroups (3 for 2 CUs): one load
+// case of a grid of up to ~60^3 makes fewer of full tiles, and the launch then
+// waits for workgroups that run alone on their CU.  Per load path, full tiles
+// against this bound: 20^3 damage 10.1 / 8.4 ms, 36^3 19.4 / 17.2, 50^3 117.9 /
+// 112.3, J2 40^3 13.5 / 11.6, 70^3 28.6 / 28.3, 100^3 69.4 / 68.6.  Bounds of 512
+// and 768 cut to single kz (96-byte rows) earlier: 40^3 13.2, 50^3 110.8 and 140.7.
+int kz_most(const Geo& g, int planes) { return std::max(1, (int)((long long)planes * g.Nzh / 384)); }
+
 template <typename K, typename... A>
 void go(K* k, int blocks, int nt, size_t sm, hipStream_t st, const A&... args)
 {
@@ -352,9 +360,11 @@ void plan(Geo& g)
     g.TY = even(g.Ny, ty);
     g.nty = (g.Ny + g.TY - 1) / g.TY;
     g.nbz = g.Nx * g.nty;
-    g.TKx = even(g.Nzh, tk);
+    g.TKx = even(g.Nzh, std::min(tk, kz_most(g, g.Ny)));
     g.nkx = (g.Nzh + g.TKx - 1) / g.TKx;
     g.nbx = g.Ny * g.nkx;
+    g.TKy = even(g.Nzh, std::min(g.TKy, kz_most(g, g.Nx)));
+    g.nky = (g.Nzh + g.TKy - 1) / g.TKy;
 }
 
 void launch_z(int beh, int mode, const Geo& g, const BPtr<T>& p, hipStream_t st, bool lin)

@@ -44,7 +44,16 @@ MAT_J2 = np.array([[400e9, 0.20, np.inf, 0, 1, 0, 0], [70e9, 0.30, 100e6, 1e9, 1
 def test_basic_x_tiles(n):
     """J2 load path over 17 kz: x tiles of 8, 5, 2 and 2 kz on 256 threads (32,
     48, 96, 128 points) and of 2 on 512 (192), the last one ragged."""
-    shape = (n, 32, 32)
+    j2_path((n, 32, 32))
+
+
+# planes * (Nz/2+1) / 384: x tiles of 2, 11 and 1 kz, y tiles of 1, 1 and 6
+@pytest.mark.parametrize("shape", [(20, 40, 44), (10, 90, 98), (100, 10, 50)])
+def test_basic_tiles_without_compile_time_kernels(shape):
+    j2_path(shape)
+
+
+def j2_path(shape):
     ids = (np.random.default_rng(7).uniform(size=shape) > 0.3).astype(np.int32)
     X0 = np.eye(6)[1]
     o = oracle.Elastic(*shape, "ep")
