@@ -437,8 +437,9 @@ struct BasicRunner {
     void fields(double* eps, double* sig)
     {
         const size_t n6 = (size_t)6 * e.N;
-        if (eps) HCHK(hipMemcpy(eps, f6, sizeof(double) * n6, hipMemcpyDeviceToHost));
-        if (sig) HCHK(hipMemcpy(sig, f6 + n6, sizeof(double) * n6, hipMemcpyDeviceToHost));
+        if (eps) e.to_host(eps, f6, sizeof(double) * n6, e.st);
+        if (sig) e.to_host(sig, f6 + n6, sizeof(double) * n6, e.st);
+        HCHK(hipStreamSynchronize(e.st));
     }
 
     // per-voxel history: equivalent plastic strain ("ep") or damage ("ed"),
@@ -446,11 +447,12 @@ struct BasicRunner {
     void state(double* ep_or_d, double* seff)
     {
         const size_t n = (size_t)e.N;
-        if (ep_or_d) HCHK(hipMemcpy(ep_or_d, f1, sizeof(double) * n, hipMemcpyDeviceToHost));
+        if (ep_or_d) e.to_host(ep_or_d, f1, sizeof(double) * n, e.st);
         if (seff) {
-            if (beh == BEH_EP) HCHK(hipMemcpy(seff, f1 + 3 * n, sizeof(double) * n, hipMemcpyDeviceToHost));
+            if (beh == BEH_EP) e.to_host(seff, f1 + 3 * n, sizeof(double) * n, e.st);
             else std::fill(seff, seff + n, 0.0);
         }
+        HCHK(hipStreamSynchronize(e.st));
     }
 };
 
