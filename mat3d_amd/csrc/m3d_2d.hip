@@ -458,6 +458,8 @@ int m3d_2d_set_load(m3d_2d* h, const double* E_ri)
         for (int c = 0; c < 3; ++c) s.E[c] = cx<double>{E_ri[2 * c], E_ri[2 * c + 1]};
         hipLaunchKernelGGL(p2::k_fill_eps, dim3(256), dim3(256), 0, s.st, s.eps, s.E[0], s.E[1], s.E[2], s.xy);
         HCHK(hipGetLastError());
+        // the fields' copies do not follow this stream, and a failed fill is this call's error
+        HCHK(hipStreamSynchronize(s.st));
         return M3D_OK;
     });
 }
