@@ -74,7 +74,7 @@ __global__ void __launch_bounds__(ZNT) M3D_BZ_ATTR kzb(Geo g, BPtr<T> p)
     const int x = t / (g.Ny / TY);
     const int y0 = (t - x * (g.Ny / TY)) * TY;
     Ctl& ctl = p.ctl[0];
-    if (ctl.done || t >= per) return;
+    if (bz_skip(ctl, blockIdx.x == 0 && threadIdx.x == 0) || t >= per) return;
     const int tid = threadIdx.x;
     const long long vox0 = ((long long)x * g.Ny + y0) * NZ;
     T* eps = p.eps + vox0 * 6;

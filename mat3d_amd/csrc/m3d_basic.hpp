@@ -259,7 +259,26 @@ __device__ __forceinline__ void bfin1(Ctl& c, const BFin& f, double (*red)[NBSUM
     }
 }
 
-// kind 2: eqVar of this iterate, diff_avr_eqVar, stop rule (:820-826)
+// Stop rule (:820-826).  It runs beside the tiles of the inverse y pass, which
+// test `done`, so the decision goes to `stop`: a word of its own that only later
+// launches test.  The next z pass tests it alone and, in its first workgroup,
+// sets `done` for the y and x passes after it.  So no launch writes a word that
+// decides whether its own workgroups run, and all waves of a workgroup agree.
+__host__ __device__ inline void bstop_rule(Ctl& c)
+{
+    if (c.err) c.stop = 3;
+    else if (c.it > 1 && fabs(c.deq) < c.tol_eq && fabs(c.dsum) < c.tol_f) c.stop = 1;
+    else if (c.it > c.cap) c.stop = 2;
+}
+// a z pass's workgroup has nothing to do; first: the launch's first thread
+__host__ __device__ inline bool bz_skip(Ctl& c, bool first)
+{
+    if (!c.stop) return false;
+    if (first) c.done = c.stop;
+    return true;
+}
+
+// kind 2: eqVar of this iterate, diff_avr_eqVar, stop rule
 __device__ __forceinline__ void bfin2(Ctl& c, const BFin& f, double* red)
 {
     const double cc = ordered_sum(f.part, f.n, red);
@@ -276,21 +295,15 @@ __device__ __forceinline__ void bfin2(Ctl& c, const BFin& f, double* red)
         c.deq = fabs(eq - c.eq_val);
         c.eq_val = eq;
         c.eqvar = eq;
-        if (c.err) c.done = 3;
-        else if (c.it > 1 && fabs(c.deq) < c.tol_eq && fabs(c.dsum) < c.tol_f) c.done = 1;
-        else if (c.it > c.cap) c.done = 2;
+        bstop_rule(c);
         publish(c, f.hs, 0);
     }
 }
 
-// a y pass's first workgroup; `done` is read before anything is written.  The
-// other workgroups of the pass read only the stop flag, which kind 2 may set
-// while they start: what they transform is then not used.
+// a y pass's first workgroup; it writes nothing that the others read
 __device__ __forceinline__ void bfin_block(Ctl& c, const BFin& f, double (*red)[NBSUM])
 {
-    const int done = c.done;
-    __syncthreads();
-    if (done) {
+    if (c.done) {
         if (f.kind == 2 && threadIdx.x == 0) publish(c, f.hs, 0);
         return;
     }

@@ -228,13 +228,13 @@ struct BasicRunner {
     // sums in pfin and applies update_old_Variable).  The iterations after the
     // start stage (itNo it0) alternate the buffers from buffer 0, so iterate
     // itNo c.it read buffer (c.it - it0 - 1) & 1.  The z pass skips a solve
-    // marked done, so the flag is cleared for it; c is the host copy of the
-    // control block after the iterations.
+    // that has stopped, so the flags are cleared for it; c is the host copy of
+    // the control block after the iterations.
     void finish(const Ctl& c, int it0)
     {
         hipStream_t st = e.st;
         cfin = c;
-        cfin.done = 0;
+        cfin.done = cfin.stop = 0;
         HCHK(hipMemcpyAsync(ctl, &cfin, sizeof cfin, hipMemcpyHostToDevice, st));
         const BPtr<double> bp = bptr_t<double>((c.it - it0 - 1) & 1);
         if (fast) bfast::launch_z<double>(beh, BMODE_FINAL, gf, bp, st, lin);
@@ -256,12 +256,13 @@ struct BasicRunner {
         }
         HCHK(hipMemcpyAsync(&c, ctl, sizeof c, hipMemcpyDeviceToHost, st));
         HCHK(hipStreamSynchronize(st));
+        c.done = c.stop;
     }
 
     // upload the control block and the state words it starts from
     void load_ctl(Ctl& c)
     {
-        c.tick = 0;
+        c.tick = c.stop = 0;
         *hs = 0;
         HCHK(hipMemcpyAsync(ctl, &c, sizeof c, hipMemcpyHostToDevice, e.st));
     }

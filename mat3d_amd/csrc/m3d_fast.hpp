@@ -1000,7 +1000,7 @@ __device__ __forceinline__ void xy_tile(const Geo& g, const Ptr<T>& p, const Ctl
 
 // solve s takes part in this pass
 template <int WHICH>
-__device__ __forceinline__ bool xy_active(const Ctl& c)
+__host__ __device__ __forceinline__ bool xy_active(const Ctl& c)
 {
     if (c.done || c.wait) return false;
     if (WHICH == BUF_CHK_CUR && !c.need_cur) return false;

@@ -239,7 +239,7 @@ __device__ __forceinline__ void store_tile(const cx<T>* sl, cx<T>* base, long lo
 }
 
 // ------------------------------------------------------------ y and x passes
-__device__ __forceinline__ bool active(const Ctl& c, int which)
+__host__ __device__ __forceinline__ bool active(const Ctl& c, int which)
 {
     return !c.done && !c.wait && (which != BUF_CHK_CUR || c.need_cur) && (which != BUF_CHK_PREV || c.need_prev);
 }

@@ -42,7 +42,7 @@ __global__ void __launch_bounds__(NT) k_zb(Geo g, BPtr<T> p)
     __shared__ double red[NBSUM + 2][NW];
     cx<T>* sl = reinterpret_cast<cx<T>*>(smem_raw);
     Ctl& ctl = p.ctl[0];
-    if (ctl.done) return;
+    if (bz_skip(ctl, blockIdx.x == 0 && threadIdx.x == 0)) return;
     const int t = fast::xcd_remap(blockIdx.x, gridDim.x);
     const int x = t / g.nty, y0 = (t - x * g.nty) * g.TY;
     const int ny = min(g.TY, g.Ny - y0), Nz = g.Nz;

@@ -62,6 +62,7 @@ struct Ctl {
     // the solve stands still until one that does (k_finA)
     int wait;
     int tick; // states published to the host since the loop began (publish)
+    int stop; // basic scheme: value of `done` that the stop rule decided on (bstop_rule)
     double sum_anchor; // sum of the dual field of the anchor (FP64)
     double sum_prev;  // sum of the dual field at iterate `it`
     double eq_val;    // eqVar at iterate eq_it
@@ -523,7 +524,7 @@ __device__ __forceinline__ void publish(Ctl& c, unsigned long long* hs, int s)
     if (!hs) return;
     c.tick += 1;
     unsigned long long v = (unsigned long long)c.tick << 8;
-    if (c.done) v |= ST_DONE;
+    if (c.done || c.stop) v |= ST_DONE;
     if (c.wait) v |= ST_WAIT;
     if (c.it >= 1 && c.dsum < NEAR_TOL * c.tol_f) v |= ST_NEAR;
     if (c.eq_it == c.it) v |= ST_CHECKED;
