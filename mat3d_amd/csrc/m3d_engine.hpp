@@ -365,7 +365,7 @@ struct XyTune {
 };
 
 struct TuneKey {
-    std::string dev; // device architecture and CU count
+    std::string dev; // device architecture and CU count, and the narrowed tiles (tile_tag)
     int nx, ny, nz, c, ns;
     bool operator<(const TuneKey& o) const
     {
@@ -460,6 +460,19 @@ inline std::string device_tag()
     const size_t c = a.find(':');
     if (c != std::string::npos) a = a.substr(0, c);
     return a + "x" + std::to_string(pr.multiProcessorCount);
+}
+
+// The tiles that a choice was timed on, where they are not the budget's (ktile
+// narrows those of short lines): a choice timed on other tiles is not found
+// under this key and timed again.  Empty for the other lengths, whose keys are
+// those of the files written before the tiles were narrowed.
+inline std::string tile_tag(const Geo& g)
+{
+    std::string s;
+    if (g.fx && g.TKx != M3D_XTILE / (g.C * g.Nx))
+        s += "+x" + std::to_string(g.TKx) + "," + std::to_string(fast::xtile_wide<float>(g.Nx, g.C));
+    if (g.fy && g.TKy != M3D_YTILE / (g.C * g.Ny)) s += "+y" + std::to_string(g.TKy);
+    return s;
 }
 
 template <typename PH>
@@ -998,7 +1011,7 @@ struct Engine {
     void tune_xy(Geo g)
     {
         g.nsolve = nsolve;
-        const TuneKey key{device_tag(), Nx, Ny, Nz, C, nsolve};
+        const TuneKey key{device_tag() + tile_tag(g), Nx, Ny, Nz, C, nsolve};
         {
             std::lock_guard<std::mutex> lk(tune_mutex());
             tune_file_load();
