@@ -117,8 +117,8 @@ int m3d_elastic_info(m3d_elastic *h, double *vol, int *strain_base, double *la0,
  * phase stops at max(tol*factor, fp32_floor), default 10), "fp32_floor"
  * (default 1e-6), "rollback" (FP32 iterations redone in FP64 when the switch
  * iterate already satisfies the stop rule within 2 x tol, default 5), "cap"
- * (iteration cap, default 2000 elastic / 500 thermal), "chunk" (iterations
- * launched per look at the state, 0 = one), "refine" (1, default: the polish iterates
+ * (iteration cap, default 2000 elastic / 500 thermal), "chunk" (accepted
+ * from 0 on, without effect: iterations are launched one at a time), "refine" (1, default: the polish iterates
  * an FP32 correction of one FP64 anchor with FP64 stop-rule sums and checks;
  * 0: plain FP64 polish iterations), "scheme" (0, default: the reference's
  * accelerated "e" loop; 1: the basic Moulinec-Suquet iteration with the load

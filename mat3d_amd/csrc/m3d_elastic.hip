@@ -48,7 +48,7 @@ struct m3d_batch {
     bool grouped = false;
     bool ran = false;
     double polish_factor = 10.0, fp32_floor = 1e-6;
-    int rollback = 5, cap = 2000, chunk = 0, max_solves = 0, refine = 1, scheme = 0, autotune = 1;
+    int rollback = 5, cap = 2000, max_solves = 0, refine = 1, scheme = 0, autotune = 1;
     double ms = 0, voxel_its = 0;
 };
 
@@ -133,7 +133,7 @@ int m3d_elastic_set_option(m3d_elastic* h, const char* key, double value)
         else if (k == "fp32_floor" && value >= 0.0) h->eng->fp32_floor = value;
         else if (k == "rollback" && value >= 0 && value <= 64) h->eng->rollback = (int)value;
         else if (k == "cap" && value >= 1) h->eng->cap = (int)value;
-        else if (k == "chunk" && value >= 0) h->eng->chunk = (int)value;
+        else if (k == "chunk" && value >= 0) return M3D_OK; // no effect
         else if (k == "refine" && (value == 0 || value == 1)) h->eng->refine = (int)value;
         else if (k == "autotune" && (value == 0 || value == 1)) h->eng->autotune = (int)value;
         else if (k == "basic_fp32" && (value == 0 || value == 1)) {
@@ -418,7 +418,7 @@ int m3d_batch_set_option(m3d_batch* b, const char* key, double value)
         else if (k == "fp32_floor" && value >= 0.0) b->fp32_floor = value;
         else if (k == "rollback" && value >= 0 && value <= 64) b->rollback = (int)value;
         else if (k == "cap" && value >= 1) b->cap = (int)value;
-        else if (k == "chunk" && value >= 0) b->chunk = (int)value;
+        else if (k == "chunk" && value >= 0) return M3D_OK; // no effect
         else if (k == "max_solves" && value >= 0) {
             b->max_solves = (int)value;
             batch_free_groups(b); // device batch sizes change
@@ -482,7 +482,6 @@ void batch_group_setup(m3d_batch* b, BatchGroup& G)
     e.fp32_floor = b->fp32_floor;
     e.rollback = b->rollback;
     e.cap = b->cap;
-    e.chunk = b->chunk;
     e.refine = b->refine;
     e.autotune = b->autotune;
 }

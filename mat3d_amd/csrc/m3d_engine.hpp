@@ -529,7 +529,6 @@ struct Engine {
     double rollback_margin = 2.0;
     double fp32_floor = 1e-6;
     int cap = 2000;
-    int chunk = 0; // iterations launched between two looks at the state (0: 1)
     int mnblk = 256;
 
     Engine(int nx, int ny, int nz, int prec) : Nx(nx), Ny(ny), Nz(nz), precision(prec)
@@ -944,7 +943,7 @@ struct Engine {
         ypass<float, 1, BUF_MAIN>(gf, pf);
     }
 
-    // The checks the next launched iterations have to hold, from the newest
+    // The checks the next launched iteration has to hold, from the newest
     // published state of the solves: none while no running solve is near its
     // stop, the current iterate's alone where every solve that is has a checked
     // iterate behind it.  A guess only: a solve that needs more than it was
@@ -961,23 +960,25 @@ struct Engine {
         return need;
     }
 
-    // Launch iterations (iter(checks), ck at a time) until every solve of the
-    // batch is done.  The host stays one group of launches ahead: it reads the
-    // state after one while the next runs, so the device does not wait for it
-    // (what was queued when the last solve ended only skips).  Plain launches:
+    // Launch iterations (iter(checks)) until every solve of the batch is done.
+    // The host stays one ahead: it reads the state after one while the next
+    // runs, so the device does not wait for it (what was queued when the last
+    // solve ended only skips).  Groups of iterations per look at the state
+    // gain nothing and stand still from the first check they do not hold to
+    // their end (64^3 FP32 + polish, groups of 1, 8, 32, 200: 2.24, 3.36, 4.88,
+    // 26.7 ms).  Plain launches:
     // they cost the host 3-4.5 us each and a kernel of the smallest grids takes
     // 4-12 us, while capturing and instantiating a graph took 50 us (12 nodes)
     // to 800 us (80 nodes) in every call, and the device 8 us between graphs.
     // The control blocks' ticks start at 0.
     template <typename Iter>
-    void run_loop(int ck, Iter&& iter, std::vector<Ctl>& hctl)
+    void run_loop(Iter&& iter, std::vector<Ctl>& hctl)
     {
         std::fill(hstate, hstate + nsolve, 0ull);
         for (unsigned long long k = 0;; ++k) {
-            const int checks = checks_for();
-            for (int i = 0; i < ck; ++i) iter(checks);
+            iter(checks_for());
             HCHK(hipGetLastError());
-            if (k > 0 && wait_ticks(st, hstate, nsolve, k * ck)) break;
+            if (k > 0 && wait_ticks(st, hstate, nsolve, k)) break;
         }
         HCHK(hipMemcpyAsync(hctl.data(), ctl, sizeof(Ctl) * nsolve, hipMemcpyDeviceToHost, st));
         HCHK(hipStreamSynchronize(st));
@@ -991,7 +992,7 @@ struct Engine {
         Ptr<T> p = ptrs<T>(g);
         launch_start<T>(g, p);
         HCHK(hipGetLastError());
-        run_loop(std::max(1, chunk), [&](int checks) { launch_iter<T>(g, p, checks); }, hctl);
+        run_loop([&](int checks) { launch_iter<T>(g, p, checks); }, hctl);
     }
 
     // anchored polish of the solves flagged corr (r and e from the anchor
@@ -1003,7 +1004,7 @@ struct Engine {
         Ptr<double> pd = ptrs<double>(gd);
         launch_start_corr(gf, pf);
         HCHK(hipGetLastError());
-        run_loop(std::max(1, chunk), [&](int checks) { launch_iter_corr(gf, pf, gd, pd, checks); }, hctl);
+        run_loop([&](int checks) { launch_iter_corr(gf, pf, gd, pd, checks); }, hctl);
     }
 
     // time the FP32 x/y pass variants on this shape (first FP32 solve); the
