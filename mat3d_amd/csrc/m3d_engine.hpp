@@ -224,7 +224,9 @@ inline bool wait_ticks(hipStream_t st, const unsigned long long* hs, int n, unsi
 // 128^3 19.6 -> 6.2, 200^3 73.4 -> 20.4; four threads take 10% more, eight the same;
 // chunks of 512 KB 40% more, of 1 MB 20% more from 128^3 on and less below.
 // Copies under DIRECT go straight to hipMemcpyAsync (48^3: 0.65 ms against 0.93),
-// as does everything where the pinned memory cannot be had.
+// as does everything where the pinned memory cannot be had, and a destination
+// that HIP knows: pinned memory takes the transfer itself (128^3 3.65 ms against
+// 5.2 through the buffers), device memory is not the host's to write.
 struct HostCopy {
     static constexpr int COPIERS = 6;
     static constexpr size_t CHUNK = (size_t)2 << 20, DIRECT = (size_t)8 << 20;
@@ -258,12 +260,21 @@ struct HostCopy {
         return false;
     }
 
+    // pinned, managed or device memory
+    static bool known(const void* dst)
+    {
+        hipPointerAttribute_t a;
+        if (hipPointerGetAttributes(&a, dst) == hipSuccess) return a.type != hipMemoryTypeUnregistered;
+        (void)hipGetLastError();
+        return false;
+    }
+
     // dst[0, bytes) = src after the work queued on st; complete when the caller
     // has synchronized st
     void operator()(void* dst, const void* src, size_t bytes, hipStream_t st)
     {
-        if (bytes < DIRECT || !ready()) {
-            HCHK(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, st));
+        if (bytes < DIRECT || known(dst) || !ready()) {
+            HCHK(hipMemcpyAsync(dst, src, bytes, hipMemcpyDefault, st));
             return;
         }
         const size_t chunk = bytes < 16 * CHUNK ? CHUNK / 2 : CHUNK;
