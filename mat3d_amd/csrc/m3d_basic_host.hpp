@@ -189,13 +189,13 @@ struct BasicRunner {
         return p;
     }
     BPtr<double> bptr() { return bptr_t<double>(); }
-    Ptr<double> yptr() { return yptr_t<double>(); }
 
     // one stage: z pass, y pass with the sums and updateE beside it, x pass, y
-    // pass with the stop rule beside it; the restart stage is a start stage (strain from HBM) that keeps itNo.  A
-    // start stage transforms [sigma | eps] and writes S6 buffer 0 (par = 1);
-    // an iteration reads S6 buffer par, transforms sigma only (the x pass
-    // keeps eps^ in Eh) and writes buffer 1 - par.
+    // pass with the stop rule beside it; the restart stage is a start stage
+    // (strain from HBM) that keeps itNo.  A start stage transforms [sigma | eps]
+    // and writes S6 buffer 0 (par = 1); an iteration reads S6 buffer par,
+    // transforms sigma only (the x pass keeps eps^ in Eh) and writes buffer
+    // 1 - par.
     template <typename T = double>
     void stage(int mode, int par)
     {

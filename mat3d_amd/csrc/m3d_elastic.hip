@@ -462,9 +462,9 @@ int m3d_batch_add(m3d_batch* b, int nx, int ny, int nz, const double* mat, const
 // independent solves.  When every shape group fits the device memory in one
 // device batch, the groups' engines run at the same time, one host thread
 // and one stream each (allocation and autotuning done first, one engine
-// after the other), so small grids and the host's polling between graph
-// replays of one group overlap the others' kernels; otherwise the groups run
-// one after another, sub-batched to fit.
+// after the other), so the short launches of small grids and the gaps between
+// them overlap the others' kernels; otherwise the groups run one after
+// another, sub-batched to fit.
 namespace {
 
 struct GroupRun {

@@ -858,8 +858,8 @@ __device__ __forceinline__ void kz_tile(const Geo& g, const Ptr<T>& p, int b, cx
     }
 }
 
-// one solve's check is needed (the check passes are captured in every
-// iteration and gated on these flags)
+// one solve's check is needed (a launch of the check passes covers every solve
+// of the batch; the ones that need none are left out by these flags)
 template <int WHICH>
 __device__ __forceinline__ bool chk_needed(const Ctl& c)
 {

@@ -7,7 +7,8 @@
 // One solve of a small grid is bound by latency: at 50^3 (250 to 450
 // workgroups) z 69 -> 17, x 63 -> 17, y 38 + 29 -> 9 + 10 us per iteration
 // against passes that transformed [sigma | eps] (12 components) in every
-// iteration; a 50^3 damage path of 2076 iterations 463 -> 163 ms.
+// iteration; a 50^3 damage path of 2076 iterations 463 -> 112 ms (with the
+// finalisers inside the y passes and the tiles of kz_most).
 #include "m3d_basic_fast.hpp"
 #include "m3d_flex.hpp"
 
