@@ -24,12 +24,13 @@
 // six solves, against the run-time-planned passes this replaces (one voxel
 // per thread through scalar loads, odd radices as direct DFTs with twiddles
 // from global memory, integer divisions by run-time widths):
-//   100^3 FP32     z update 835 -> 132 us (4.4 TB/s), x with the Green step
-//                  378 -> 77 us (3.8 TB/s), y 238 -> 48 us (6.1 TB/s)
-//   45x50x56 FP64  z 237 -> 41, x 131 -> 30, y 82 -> 20 us
-//   96^3 thermal   (three solves, FP64) z 103 -> 69, x 88 -> 37, y 54 -> 26 us
-// A homogenization: 100^3 FP32 94 -> 23 ms, 45x50x56 FP64 17.6 -> 4.6 ms,
-// 96^3 thermal 10.2 -> 6.0 ms.
+//   100^3 FP32     z update 835 -> 129 us, x with the Green step 378 -> 74, y
+//                  238 -> 48 (averages of a homogenization; while all six
+//                  solves run 151 us, 3.9 TB/s, 84, 3.5, and 55, 5.3)
+//   45x50x56 FP64  z 237 -> 42, x 131 -> 31, y 82 -> 21 us
+//   96^3 thermal   (three solves, FP64) z 103 -> 74, x 88 -> 39, y 54 -> 27 us
+// A homogenization, with the check passes left out where no solve needs them:
+// 100^3 FP32 101 -> 24 ms, 45x50x56 FP64 16.9 -> 3.9, 96^3 thermal 10.4 -> 5.2.
 #pragma once
 #include "m3d_fast.hpp"
 
